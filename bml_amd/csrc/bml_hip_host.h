@@ -18,6 +18,8 @@ struct bml_hip_aux {
     int touched_hint;      /* distinct columns per row seen the last time this
                               matrix was squared (0 = unknown) */
     int hint_max_nnz;      /* its longest row at that time */
+    int len_hint;          /* stats not valid: about the longest row (0 = unknown;
+                              launch shapes only) */
 };
 
 /* Record an error.  In BML_HIP_ERRORS_EXIT mode prints it the way bml's
@@ -49,6 +51,8 @@ int bmlh_block_engine_setting(void);
 /* the real scalar s as one element of precision prec, into buf (16 bytes) */
 void bmlh_put_scalar(int prec, double s, void *buf);
 struct bml_hip_aux *bmlh_aux_new(void);
+/* the row statistics no longer hold: rows may have grown by `more` entries */
+void bmlh_stats_stale(struct bml_hip_aux *aux, int more);
 void bmlh_set_stats(struct bml_hip_aux *aux, const bmlhip_status *st);
 /* The row-major dense N x N host array (malloc'd) of an ellpack_hip or
  * ellblock_hip matrix A, its elements cast to precision; N into *N_out. */

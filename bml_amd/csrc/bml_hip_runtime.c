@@ -144,7 +144,17 @@ void bmlh_set_stats(struct bml_hip_aux *aux, const bmlhip_status *st)
         aux->total_nnz = st->total_nnz;
     } else {
         aux->stats_valid = 0;
+        aux->len_hint = 0;
     }
+}
+
+void bmlh_stats_stale(struct bml_hip_aux *aux, int more)
+{
+    if (aux->stats_valid)
+        aux->len_hint = aux->max_nnz;
+    if (aux->len_hint > 0)
+        aux->len_hint += more;
+    aux->stats_valid = 0;
 }
 
 /* ---- public runtime API ------------------------------------------------ */

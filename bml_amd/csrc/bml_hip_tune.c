@@ -31,7 +31,102 @@
 #include <stdlib.h>
 #include <string.h>
 
-void bmlh_pick_spgemm(int precision, int N, int max_a, int max_b, int touched_hint,
+/* Shape of the direct-index kernel (hip/rowdir.hip), 0 when its LDS cannot
+ * hold one row.
+ *
+ * GROUP lanes per row: enough for a row of B in one chunk (rows of up to 8,
+ * 16 or 32 entries share a wavefront), wider while the matrix has too few
+ * rows to fill the GPU's 1024 SIMDs twice over; up to five 64-lane chunks a
+ * step.  W wavefronts per block and the blocks per CU follow the LDS: the
+ * block needs 8 bytes per 32 reachable columns, and each row sizeof(T) + 2 per
+ * column that any row of the block touches (15% more for each further row: on
+ * a lattice a step along the fast axis adds the ball's cross-section); the W with the most wavefronts per CU is taken, the larger
+ * of equals (its rows share more of the index).  A block whose rows touch
+ * more than that forms them in several passes, so a wrong guess costs time
+ * only; without a hint the bound min(span, max_a * max_b) is far above the
+ * truth, and 3000 columns are the most that are provided for.
+ * Rows so short that all columns fit are indexed by the column itself. */
+static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long long est,
+                       int known, int grows, bmlh_spgemm_shape *out)
+{
+    if (N <= 0 || span <= 0)
+        return 0;
+    int g = 8;
+    while (g < 64 && (g < max_b || (long long) N * g < 64 * 2048))
+        g <<= 1;
+    int nch = (max_b + g - 1) / g;
+    if (nch > 5)
+        nch = (nch + (nch + 4) / 5 - 1) / ((nch + 4) / 5);
+    if (nch < 1)
+        nch = 1;
+    if (est > span)
+        est = span;
+    const long long per = (long long) es + 2;
+    const int dense = span * per <= 6 * 1024 || (2 * est >= span && span * per <= 20 * 1024);
+    if (!known && est > 3000)
+        est = 3000;
+    /* growing rows touch more columns for their length each time (a ball of
+     * radius r squared has radius 2r) */
+    if (grows && est + est / 2 <= span)
+        est += est / 2;
+    const long long words = span / 32 + 2;
+    const long long cu = 160 * 1024;
+    int best = 0, best_waves = 0;
+    long long best_lds = 0;
+    for (int w = 8; w >= 1; w--) {
+        const int rb = w * (64 / g);
+        if (w > 1 && (long long) N < 256ll * rb)
+            continue; /* fewer blocks than CUs */
+        long long D = est + est * 15 * (rb - 1) / 100 + 32;
+        if (dense || D > span)
+            D = span;
+        long long need = 8 * words + 64 + (span > 65536 ? 4 * D + 16 : 0) + 64ll * w * (long long) es +
+                         rb * (D * per + 32);
+        /* the lists of the symbolic phase */
+        const long long list = (long long) rb * max_a < span ? (long long) rb * max_a : span;
+        const long long low = 12 * words + 128 + 4 * list + 1024;
+        if (need < low)
+            need = low;
+        if (need > cu)
+            continue;
+        long long k = cu / ((need + 1279) / 1280 * 1280);
+        if (k * w > 16)
+            k = 16 / w;
+        if (k * w > best_waves) {
+            best = w;
+            best_waves = (int) (k * w);
+            /* the whole share of the CU (allocated in 1280 bytes): est may
+             * be low, above all while rows grow */
+            best_lds = cu / k / 1280 * 1280;
+        }
+    }
+    if (!best)
+        return 0;
+    out->engine = BMLHIP_ROW_DIRECT;
+    out->group = g;
+    out->bucket = nch;
+    out->waves = best;
+    out->table = (int) best_lds;
+    out->wrows = span;
+    /* two rows share too few rows of B to pay for listing them */
+    out->wbits = dense ? BMLHIP_DIR_DENSE
+                       : (best * (64 / g) <= 2 && max_a <= 96 ? BMLHIP_DIR_OWN : BMLHIP_DIR_LIST);
+    if (best * (64 / g) == 1 && !dense)
+        out->wbits = BMLHIP_DIR_OWN;
+    return 1;
+}
+
+static int shape_from_env(void)
+{
+    static const char *const names[] = { "BML_HIP_GROUP", "BML_HIP_TABLE", "BML_HIP_BUCKET",
+                                         "BML_HIP_WAVES", "BML_HIP_LDS_BUDGET" };
+    for (size_t k = 0; k < sizeof names / sizeof names[0]; k++)
+        if (getenv(names[k]))
+            return 1;
+    return 0;
+}
+
+void bmlh_pick_spgemm(int precision, int N, int span, int max_a, int max_b, int touched_hint,
                       int hint_max_a, int flags, bmlh_spgemm_shape *out)
 {
     const int square = flags & BMLH_PICK_SQUARE;
@@ -206,6 +301,11 @@ void bmlh_pick_spgemm(int precision, int N, int max_a, int max_b, int touched_hi
     /* contiguous rows per XCD cut the HBM fetch of the lattice X^2 5x but
      * ran 1.3x slower than the hardware's round-robin order */
     out->remap = (e = getenv("BML_HIP_XCD_REMAP")) ? atoi(e) : 0;
+    /* the exact engine's work goes to the direct-index kernel wherever its
+     * LDS holds a row (a shape from the environment is the hash kernels') */
+    if (engine == BMLHIP_ROW_EXACT && !shape_from_env())
+        pick_direct(bmlh_elem_size(precision), N, span, max_a, max_b, est, touched_hint > 0,
+                    touched_hint > 0 && 20 * max_a > 21 * hint_max_a, out);
 }
 
 /* ---- measured shapes ------------------------------------------------------
@@ -367,7 +467,7 @@ void bmlh_tuned_spgemm(int precision, int N, int max_a, int max_b, int touched_h
                        int hint_max_a, int flags, bmlh_spgemm_shape *out, bmlh_measure_fn fn,
                        void *ctx)
 {
-    bmlh_pick_spgemm(precision, N, max_a, max_b, touched_hint, hint_max_a, flags, out);
+    bmlh_pick_spgemm(precision, N, N, max_a, max_b, touched_hint, hint_max_a, flags, out);
     tune_env();
     if (!g_tune || !fn || N <= 0)
         return;
@@ -421,6 +521,19 @@ void bmlh_tuned_spgemm(int precision, int N, int max_a, int max_b, int touched_h
             c.table = (k ? t0 * 3 / 2 : t0 * 3 / 4) / 64 * 64;
             if (c.table >= 256)
                 try_shape(&c, &best, &best_ms, fn, ctx);
+        }
+    } else if (out->engine == BMLHIP_ROW_DIRECT) {
+        /* wavefronts per block and the LDS that goes with them */
+        const int w0 = best.waves, t0 = best.table;
+        for (int w = w0 / 2; w <= 2 * w0 && w <= 8; w *= 2) {
+            if (w < 1 || w == w0)
+                continue;
+            c = best;
+            c.waves = w;
+            c.table = (int) ((long long) t0 * w / w0);
+            if (c.table > 160 * 1024)
+                c.table = 160 * 1024;
+            try_shape(&c, &best, &best_ms, fn, ctx);
         }
     } else {
         static const int bk[] = {2, 4, 8};

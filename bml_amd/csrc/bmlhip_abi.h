@@ -152,6 +152,17 @@ typedef struct bmlhip_spgemm_args {
 #define BMLHIP_ROW_WINDOW 2 /* x2 only (A = B): waves wavefronts per row add
                                into a dense LDS window of 2^wbits columns at a
                                time; rows come out sorted by column */
+#define BMLHIP_ROW_DIRECT 3 /* the exact engine's sums and order on directly
+                               indexed LDS accumulators (hip/rowdir.hip): group
+                               lanes per row, bucket = chunks of a row of B per
+                               step, waves = wavefronts per block, table = LDS
+                               bytes per block, wrows = columns a block's rows
+                               can reach, wbits = how they are numbered */
+#define BMLHIP_DIR_LIST 0  /* the touched ones, found from the list of the rows
+                              of B that the block's rows name */
+#define BMLHIP_DIR_DENSE 1 /* all of them: a column is its own slot */
+#define BMLHIP_DIR_OWN 2   /* the touched ones, each row's found from its own
+                              rows of B */
 /* scratch slots of the window engine: packed rows, window offsets, window
  * masks, per-row norms */
 #define BMLHIP_WIN_PACK_SLOT 12

@@ -53,7 +53,11 @@ static int same_shape(const bml_matrix_ellpack_hip_t *A, const bml_matrix_ellpac
 
 static int max_nnz_of(const bml_matrix_ellpack_hip_t *A)
 {
-    return (A->aux && A->aux->stats_valid) ? A->aux->max_nnz : A->M;
+    if (!A->aux)
+        return A->M;
+    if (A->aux->stats_valid)
+        return A->aux->max_nnz;
+    return A->aux->len_hint > 0 && A->aux->len_hint < A->M ? A->aux->len_hint : A->M;
 }
 
 static bml_matrix_ellpack_hip_t *alloc_ell(int prec, int N, int M, int mode, int zero,
@@ -684,7 +688,7 @@ void bml_add_identity_ellpack_hip(bml_matrix_ellpack_hip_t *A, double beta, doub
                                            A->nnz, NULL, beta, threshold, 1), what))
         return;
     finish_into(what, A);
-    A->aux->stats_valid = 0;
+    bmlh_stats_stale(A->aux, 1);
 }
 
 void bml_scale_add_identity_ellpack_hip(bml_matrix_ellpack_hip_t *A, double alpha, double beta,
@@ -699,7 +703,7 @@ void bml_scale_add_identity_ellpack_hip(bml_matrix_ellpack_hip_t *A, double alph
                                            A->nnz, s, beta, threshold, 1), what))
         return;
     finish_into(what, A);
-    A->aux->stats_valid = 0;
+    bmlh_stats_stale(A->aux, 1);
 }
 
 void bml_scale_inplace_ellpack_hip(const void *scale_factor, bml_matrix_ellpack_hip_t *A)
@@ -724,7 +728,7 @@ void bml_threshold_ellpack_hip(bml_matrix_ellpack_hip_t *A, double threshold)
         return;
     bmlhip_status st;
     bmlh_finish(what, &st);
-    A->aux->stats_valid = 0;
+    bmlh_stats_stale(A->aux, 0);
     A->aux->touched_hint = 0;
 }
 
@@ -784,7 +788,7 @@ void bml_normalize_ellpack_hip(bml_matrix_ellpack_hip_t *A, double mineval, doub
                                            A->nnz, s, maxeval / span, 0.0, 1), what))
         return;
     finish_into(what, A);
-    A->aux->stats_valid = 0;
+    bmlh_stats_stale(A->aux, 1);
 }
 
 /* ---- Matrix Market files -------------------------------------------------- */

@@ -23,7 +23,7 @@
 // are listed for a second pass that runs the same code on a large table in
 // global memory (one wavefront per row), so no input is ever refused.
 #include "../bmlhip_abi.h"
-#include "devtypes.h"
+#include "rowprod.h"
 
 #include <limits.h>
 #include <type_traits>
@@ -37,83 +37,15 @@ namespace {
 
 constexpr int EMPTY = -1;
 
-// bml_matrix_precision_t of an element type
-template <typename T> struct PrecOf;
-template <> struct PrecOf<float> { static constexpr int value = 1; };
-template <> struct PrecOf<double> { static constexpr int value = 2; };
-template <> struct PrecOf<cf32> { static constexpr int value = 3; };
-template <> struct PrecOf<cf64> { static constexpr int value = 4; };
 // global-table pass: at most this many blocks, and at most this many bytes
 // of tables in total
 constexpr int FALLBACK_BLOCKS = 256;
 constexpr size_t FALLBACK_BYTES = (size_t) 1 << 30;
 
-template <typename T>
-__device__ __forceinline__ T shfl_any(T v, int src) {
-    static_assert(sizeof(T) % 4 == 0, "element must be a multiple of 4 bytes");
-    union U {
-        T t;
-        int w[sizeof(T) / 4];
-    } u, r;
-    u.t = v;
-#pragma unroll
-    for (int k = 0; k < (int) (sizeof(T) / 4); k++) r.w[k] = __shfl(u.w[k], src, 64);
-    return r.t;
-}
-
 __device__ __forceinline__ unsigned hash_slot(int col, int tbits) {
     return ((unsigned) col * 0x9E3779B1u) >> (32 - tbits);
 }
 
-
-struct SpParams {
-    int N, MA, MB, MC, kind;
-    const void *Av;
-    const int *Ai, *An;
-    const void *Bv;
-    const int *Bi, *Bn;
-    void *Cv;
-    int *Ci, *Cn;
-    double thr;
-    double *rowtr;  // [2*N]: per-row tr X and tr X^2 contributions (x2)
-    bmlhip_status *st;
-    int *ovf;         // rows handed to the global-table pass
-    const int *skip;  // when set and nonzero, the launch does nothing
-    int4 *rowstat;    // [N]: (kept, distinct columns, products, nnz of A's row),
-                      // kept = -1 for a skipped row; reduced by k_row_stats
-    int remap;        // XCD-aware block-to-row order
-    int sym;          // symmetric x2: rows form only the columns k >= i
-    // batched systems: row i belongs to system row_sys[i]; rows of systems
-    // with sys_done set are skipped (both NULL: one system)
-    const int *row_sys, *sys_done;
-    // fuse: C <- beta*C + alpha*(A*B), merged in the epilogue
-    int fuse;
-    double alpha, beta;
-    // batched work queue (NULL: one block per row): the rows to form are
-    // qlist[0 .. qinfo[0]), taken with the cursor qinfo[1]
-    const int *qlist;
-    int *qinfo;
-};
-
-// Broadcast lane src's value to the caller's lanes.  With one group per
-// wavefront src is wave-uniform and a scalar readlane does it.
-template <int GROUP, typename T>
-__device__ __forceinline__ T bcast(T v, int src) {
-    if constexpr (GROUP == 64) {
-        static_assert(sizeof(T) % 4 == 0, "element must be a multiple of 4 bytes");
-        union U {
-            T t;
-            int w[sizeof(T) / 4];
-        } u, r;
-        u.t = v;
-#pragma unroll
-        for (int k = 0; k < (int) (sizeof(T) / 4); k++)
-            r.w[k] = __builtin_amdgcn_readlane(u.w[k], src);
-        return r.t;
-    } else {
-        return shfl_any(v, src);
-    }
-}
 
 // A step holds up to NCH GROUP-wide chunks of a row of B in registers.
 constexpr int NCH = 3;
@@ -3369,7 +3301,7 @@ int sp2_window_typed(int N, int M, void *Xv, int *Xi, int *Xn, double thr, int w
 
 template <typename T>
 int spgemm_typed(const bmlhip_spgemm_args *a) {
-    if (a->fuse && (a->engine != BMLHIP_ROW_EXACT || a->batch || a->sym || a->d_ws ||
+    if (a->fuse && ((a->engine != BMLHIP_ROW_EXACT && a->engine != BMLHIP_ROW_DIRECT) || a->batch || a->sym || a->d_ws ||
                     a->d_Cv == a->d_Av || a->d_Cv == a->d_Bv || a->kind == 2))
         return fail_msg(2, "fused multiply: exact engine, one system, C distinct from A and B");
     if (!a->d_ws && !a->fuse && a->engine == BMLHIP_ROW_WINDOW && a->kind == 0 && a->d_Av == a->d_Bv &&
@@ -3405,6 +3337,7 @@ int spgemm_typed(const bmlhip_spgemm_args *a) {
     p.st = bmlhip_status_dev();
     p.row_sys = a->batch ? a->batch->d_row_sys : nullptr;
     p.sys_done = a->batch ? a->batch->d_done : nullptr;
+    p.row_off = a->batch ? a->batch->d_row_off : nullptr;
     p.remap = a->remap;
     p.sym = 0;
     p.fuse = a->fuse;
@@ -3471,12 +3404,17 @@ int spgemm_typed(const bmlhip_spgemm_args *a) {
     // finished systems return at once): on the 512-system batch at hopping
     // -0.1 they ran 147 solves/s so, against 129 persistent (each take waits
     // for the listed row's index before the row's loads can start).
-    if (a->batch && a->batch->d_list && !(a->group == 64 && a->waves > 1)) {
+    // The direct-index kernel takes consecutive rows: its blocks share an
+    // index of the columns their rows reach.
+    const bool direct = a->engine == BMLHIP_ROW_DIRECT;
+    if (a->batch && a->batch->d_list && !direct && !(a->group == 64 && a->waves > 1)) {
         p.qlist = a->batch->d_list;
         p.qinfo = a->batch->d_qinfo;
     }
     int *fill = nullptr;
-    if (sym) {
+    if (direct) {
+        rc = launch_rowdir<T>(p, a->group, a->bucket, a->waves, a->table, a->wrows, a->wbits, s);
+    } else if (sym) {
         fill = (int *) bmlhip_scratch_zeroed(BMLHIP_SYMFILL_SLOT, sizeof(int) * (size_t) (a->N + 1));
         if (!fill) return fail_msg(4, "scratch allocation failed");
         p.sym = 1;

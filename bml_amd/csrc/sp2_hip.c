@@ -111,7 +111,8 @@ static int measure_sp2(const bmlh_spgemm_shape *sh, void *ctx, double *ms)
 static void sp2_shape(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpack_hip_t **X2p,
                       double threshold, int sym, bmlh_spgemm_shape *sh)
 {
-    const int mx = X->aux->stats_valid ? X->aux->max_nnz : X->M;
+    const int mx = X->aux->stats_valid ? X->aux->max_nnz
+                   : X->aux->len_hint > 0 && X->aux->len_hint < X->M ? X->aux->len_hint : X->M;
     sp2_tune_ctx c = { X, X2p, threshold, sym };
     bmlh_tuned_spgemm(X->matrix_precision, X->N, mx, mx, X->aux->touched_hint,
                       X->aux->hint_max_nnz, BMLH_PICK_SQUARE, sh, measure_sp2, &c);
@@ -335,7 +336,7 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
         if (!bmlh_finish_sync(what, &s))
             goto out;
     }
-    X->aux->stats_valid = 0; /* row totals recomputed on demand */
+    bmlh_stats_stale(X->aux, 0); /* row totals recomputed on demand */
     r.iterations = st.it;
     r.converged = st.done;
     r.trace_x = st.trx;
@@ -592,13 +593,24 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
         single = 1;
     }
 
+    /* the columns 64 consecutive rows can reach: from a system's first row to
+     * the end of the system 63 rows past its last */
+    int span = 0;
+    for (int s = 0, e = 0, lo = 0, hi = 0; s < nsys; s++) {
+        /* lo: rows before system s; hi: rows up to the end of system e - 1 */
+        while (e < nsys && (e <= s || hi < lo + H[s]->N + 63))
+            hi += H[e++]->N;
+        if (hi - lo > span)
+            span = hi - lo;
+        lo += H[s]->N;
+    }
     int touched = 0, hint_max = 0, stats[2] = { 0, 0 }, alldone[2] = { 0, 0 };
     for (int it = 0; it < o.maxit; it++) {
         bml_matrix_ellpack_hip_t *cur = single ? Xs : Xc, *cur2 = single ? X2s : X2c;
         const int mx = cur->aux->stats_valid ? cur->aux->max_nnz : cur->M;
         bmlh_spgemm_shape sh;
-        bmlh_pick_spgemm(cur->matrix_precision, N, mx, mx, touched, hint_max, BMLH_PICK_SQUARE,
-                         &sh);
+        bmlh_pick_spgemm(cur->matrix_precision, N, span, mx, mx, touched, hint_max,
+                         BMLH_PICK_SQUARE, &sh);
         if (o.graph) {
             /* replay the iteration as a graph; capture anew when the launch
              * shape or the precision changes (the first pass runs eagerly so
@@ -664,6 +676,7 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
                                                 X[s]->index, X[s]->nnz, -row_off[s]), what))
                 goto out;
             X[s]->aux->stats_valid = 0;
+            X[s]->aux->len_hint = Xc->aux->stats_valid ? Xc->aux->max_nnz : 0;
         }
         bmlhip_status st;
         if (!bmlh_finish_sync(what, &st))
