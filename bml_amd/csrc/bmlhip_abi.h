@@ -34,6 +34,8 @@ typedef struct bmlhip_status {
     long long prof_touched[5];  /* distinct columns before thresholding */
     long long prof_streamed[5]; /* entries of B's rows read (the products, unless
                                    several output rows share each read) */
+    int tail_done;              /* blocks of the running k_tail that have ended */
+    int pad_;
 } bmlhip_status;
 
 /* Per-row records: kernels store (kept, distinct, products, nnz of A's row)
@@ -85,6 +87,52 @@ int bmlhip_status_reset(void);
 /* reset everything, overflow fields included */
 int bmlhip_status_clear_errors(void);
 int bmlhip_status_fetch(bmlhip_status *host);
+
+/* Device state of one SP2 solve. */
+typedef struct bmlhip_sp2_state {
+    int it;          /* iterations done */
+    int done;        /* converged: later iterations are no-ops */
+    int branch;      /* last branch: 0 X <- X^2, 1 X <- 2X - X^2 */
+    int max_nnz;     /* X's longest row after the last update */
+    int max_touched; /* longest pre-threshold row of the last product */
+    int max_nnz_x2;  /* longest row of the last X^2 */
+    double ab[2];    /* alpha, beta of the pending add */
+    double trx, trx2, norm; /* last tr X, tr X^2, ||X - X^2||_F */
+} bmlhip_sp2_state;
+
+/* What a solve does with the sums at the end of an operation (hip/tail.hip):
+ * after x2 the branch decision, after the add the convergence test, for one
+ * system or a batch; and the pinned host memory the results go to. */
+#define BMLHIP_TAIL_NONE 0
+#define BMLHIP_TAIL_DECIDE 1
+#define BMLHIP_TAIL_CHECK 2
+#define BMLHIP_TAIL_DECIDE_BATCH 3
+#define BMLHIP_TAIL_CHECK_BATCH 4
+typedef struct bmlhip_sp2_tail {
+    int op;
+    bmlhip_sp2_state *state; /* one system */
+    double nocc, tol;
+    double *hist;
+    int maxit;
+    int touched; /* CHECK: record the longest pre-threshold row too */
+    const double *d_nocc; /* batch: [nsys] arrays, and the two counters */
+    double *ab, *norm;
+    int *branch, *it, *stats, *alldone;
+} bmlhip_sp2_tail;
+typedef struct bmlhip_host {
+    bmlhip_status status;
+    bmlhip_sp2_state state; /* after the last CHECK */
+    int stats[2], alldone;  /* after the last CHECK_BATCH */
+} bmlhip_host;
+bmlhip_host *bmlhip_host_dev(void);
+/* the last queued operation wrote its status to the host and left the status
+ * block clear */
+void bmlhip_status_published(void);
+/* the status block is clear for an operation that ends with k_tail */
+int bmlhip_status_ready(void);
+/* wait, then the state of the last BMLHIP_TAIL_CHECK / _CHECK_BATCH */
+int bmlhip_sp2_state_fetch(bmlhip_sp2_state *st);
+int bmlhip_sp2_stats_fetch(int stats[2], int *alldone);
 
 /* ---- ELLPACK kernels (hip/ellpack.hip) ---------------------------------- */
 
@@ -146,6 +194,8 @@ typedef struct bmlhip_spgemm_args {
                          product's epilogue (exact engine, kind 0 or 1, one
                          system, C distinct from A and B) */
     double alpha, beta;
+    const bmlhip_sp2_tail *sp2; /* not NULL: the solve's decision, taken where
+                                   the traces are complete */
 } bmlhip_spgemm_args;
 #define BMLHIP_ROW_EXACT 0
 #define BMLHIP_ROW_UNORDERED 1
@@ -195,10 +245,12 @@ int bmlhip_rowstat_reduce(int N, int MC, int what, int prof, const int *d_skip);
 int bmlhip_is_symmetric(int prec, int N, int M, const void *d_Av, const int *d_Ai,
                         const int *d_An, int *symmetric);
 /* as bmlhip_add with alpha = d_ab[0], beta = d_ab[1] read on the device and
- * nothing done when *d_skip != 0 */
+ * nothing done when *d_skip != 0; sp2 (or NULL): the solve's convergence
+ * test, taken where the norm is complete */
 int bmlhip_add_dev(int prec, int N, int MA, void *d_Av, int *d_Ai, int *d_An,
                    int MB, const void *d_Bv, const int *d_Bi, const int *d_Bn,
-                   const double *d_ab, double threshold, int mode, const int *d_skip);
+                   const double *d_ab, double threshold, int mode, const int *d_skip,
+                   const bmlhip_sp2_tail *sp2);
 
 /* ---- profiling window ----------------------------------------------------- */
 /* begin: zero the prof_* counters and time every row-product launch with HIP
@@ -211,17 +263,6 @@ void bmlhip_prof_mark_begin(int prec);
 void bmlhip_prof_mark_end(void);
 
 /* ---- SP2 (hip/sp2.hip) ---------------------------------------------------- */
-/* Device state of one SP2 solve. */
-typedef struct bmlhip_sp2_state {
-    int it;          /* iterations done */
-    int done;        /* converged: later iterations are no-ops */
-    int branch;      /* last branch: 0 X <- X^2, 1 X <- 2X - X^2 */
-    int max_nnz;     /* X's longest row after the last update */
-    int max_touched; /* longest pre-threshold row of the last product */
-    int max_nnz_x2;  /* longest row of the last X^2 */
-    double ab[2];    /* alpha, beta of the pending add */
-    double trx, trx2, norm; /* last tr X, tr X^2, ||X - X^2||_F */
-} bmlhip_sp2_state;
 /* After x2 (status scalars 0,1 hold tr X, tr X^2): choose the branch that
  * lands tr closer to nocc, store alpha/beta, record history[it*4..]. */
 int bmlhip_sp2_decide(bmlhip_sp2_state *d_state, double nocc, double *d_hist, int maxit);
@@ -253,7 +294,8 @@ void bmlhip_graph_destroy(void *exec);
  * b->d_ab, per-system norms into b->d_norm2 */
 int bmlhip_add_batch(int prec, int N, int MA, void *d_Av, int *d_Ai, int *d_An,
                      int MB, const void *d_Bv, const int *d_Bi, const int *d_Bn,
-                     double threshold, int mode, const bmlhip_batch *b);
+                     double threshold, int mode, const bmlhip_batch *b,
+                     const bmlhip_sp2_tail *sp2);
 /* per-system Gershgorin bounds of a batched matrix -> d_emin, d_emax [nsys] */
 int bmlhip_gershgorin_batch(int prec, int N, int M, const void *d_Av, const int *d_Ai,
                             const int *d_An, const bmlhip_batch *b, double *d_emin,
@@ -261,13 +303,6 @@ int bmlhip_gershgorin_batch(int prec, int N, int M, const void *d_Av, const int 
 /* per-system X0 = (emax I - X)/(emax - emin) in place (normalize) */
 int bmlhip_normalize_batch(int prec, int N, int M, void *d_Av, int *d_Ai, int *d_An,
                            const bmlhip_batch *b, const double *d_emin, const double *d_emax);
-/* per-system branch decision / convergence test (after x2 / after add);
- * d_alldone counts the finished systems; d_stats[0] receives the product's
- * longest pre-threshold row, d_stats[1] the longest row of X after the add */
-int bmlhip_sp2_decide_batch(const bmlhip_batch *b, const double *d_nocc, int *d_branch,
-                            int *d_stats);
-int bmlhip_sp2_check_batch(const bmlhip_batch *b, double tol, int maxit, int *d_it,
-                           double *d_norm, int *d_alldone, int *d_stats);
 /* copy rows from (N, MA) to (N, MB) adding col_shift to every column index */
 int bmlhip_copy_rows_shift(int prec, int N, int MA, const void *d_Av, const int *d_Ai,
                            const int *d_An, int MB, void *d_Bv, int *d_Bi, int *d_Bn,

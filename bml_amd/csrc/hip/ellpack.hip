@@ -24,6 +24,7 @@
 // global memory (one wavefront per row), so no input is ever refused.
 #include "../bmlhip_abi.h"
 #include "rowprod.h"
+#include "tail.h"
 
 #include <limits.h>
 #include <type_traits>
@@ -2209,88 +2210,12 @@ __global__ __launch_bounds__(64) void k_spgemm_global(SpParams p, unsigned tsize
     }
 }
 
-// Reduces per-row records (kept, distinct, products, nnz of A's row), kept
-// = -1 marking a skipped row, into the status block.  `what` selects:
-// BMLHIP_RS_OVF_KEPT / BMLHIP_RS_OVF_DIST count the rows whose kept /
-// distinct count exceeds MC (and the first of them), BMLHIP_RS_STORED the
-// largest and total stored row (kept capped at MC), BMLHIP_RS_PROF the
-// profiling sums of precision `prof`.  One set of atomics per block.
+// The row records into the status block (operations that end without k_tail).
 __global__ __launch_bounds__(256) void k_reduce_rowstat(const int4 *rs, int N, int MC, int what,
                                                         int prof, const int *skip,
                                                         bmlhip_status *st) {
     if (skip && *skip) return;
-    int ovf = 0, first = INT_MAX, mx = 0, mt = 0;
-    unsigned long long tot = 0, prods = 0, rows = 0, innz = 0, dist = 0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < N; i += gridDim.x * 256) {
-        const int4 r = rs[i];
-        if (r.x < 0) continue;
-        const int stored = r.x < MC ? r.x : MC;
-        if (((what & BMLHIP_RS_OVF_KEPT) && r.x > MC) || ((what & BMLHIP_RS_OVF_DIST) && r.y > MC)) {
-            ovf++;
-            first = i < first ? i : first;
-        }
-        mx = stored > mx ? stored : mx;
-        mt = r.y > mt ? r.y : mt;
-        tot += (unsigned long long) stored;
-        prods += (unsigned long long) (unsigned) r.z;
-        rows++;
-        innz += (unsigned long long) r.w;
-        dist += (unsigned long long) r.y;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        ovf += __shfl_down(ovf, off, 64);
-        const int f = __shfl_down(first, off, 64);
-        first = f < first ? f : first;
-        const int a = __shfl_down(mx, off, 64);
-        mx = a > mx ? a : mx;
-        const int b = __shfl_down(mt, off, 64);
-        mt = b > mt ? b : mt;
-        tot += __shfl_down(tot, off, 64);
-        prods += __shfl_down(prods, off, 64);
-        rows += __shfl_down(rows, off, 64);
-        innz += __shfl_down(innz, off, 64);
-        dist += __shfl_down(dist, off, 64);
-    }
-    __shared__ int si[4][4];
-    __shared__ unsigned long long sl[4][5];
-    const int w = threadIdx.x / 64;
-    if ((threadIdx.x & 63) == 0) {
-        si[w][0] = ovf; si[w][1] = first; si[w][2] = mx; si[w][3] = mt;
-        sl[w][0] = tot; sl[w][1] = prods; sl[w][2] = rows; sl[w][3] = innz; sl[w][4] = dist;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < 4; k++) {
-            ovf += si[k][0];
-            first = si[k][1] < first ? si[k][1] : first;
-            mx = si[k][2] > mx ? si[k][2] : mx;
-            mt = si[k][3] > mt ? si[k][3] : mt;
-            tot += sl[k][0]; prods += sl[k][1]; rows += sl[k][2]; innz += sl[k][3]; dist += sl[k][4];
-        }
-        if (ovf) {
-            atomicAdd(&st->m_overflow_rows, ovf);
-            atomicMin(&st->first_m_overflow, first);
-        }
-        if ((what & BMLHIP_RS_STORED) && rows) {
-            atomicMax(&st->max_nnz, mx);
-            atomicAdd((unsigned long long *) &st->total_nnz, tot);
-        }
-        if ((what & BMLHIP_RS_PROF) && rows) {
-            atomicMax(&st->max_touched, mt);
-            atomicAdd((unsigned long long *) &st->prof_products[prof], prods);
-            atomicAdd((unsigned long long *) &st->prof_rows[prof], rows);
-            atomicAdd((unsigned long long *) &st->prof_in_nnz[prof], innz);
-            atomicAdd((unsigned long long *) &st->prof_out_nnz[prof], tot);
-            atomicAdd((unsigned long long *) &st->prof_touched[prof], dist);
-            if (!(what & BMLHIP_RS_OWN_STREAM))
-                atomicAdd((unsigned long long *) &st->prof_streamed[prof], prods);
-        }
-    }
-}
-
-inline int rowstat_blocks(int N) {
-    const int b = (N + 2047) / 2048;
-    return b < 1 ? 1 : (b > 240 ? 240 : b);
+    reduce_rowstat(rs, N, MC, what, prof, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256, st);
 }
 
 // Deterministic sum of n doubles (fixed partition, fixed tree).
@@ -2334,8 +2259,6 @@ __global__ __launch_bounds__(1024) void k_minmax(const double *x, const double *
     }
 }
 
-// Per-system sums of x over row ranges [off[s], off[s+1]) (fixed partition
-// and tree: deterministic); systems with done[s] set are left alone.
 // Work queue of a batched iteration.  k_batch_scan (one block): act_off[s]
 // = rows of the unfinished systems before s, qinfo = (rows listed, 0, 0,
 // systems left).  k_batch_fill (one block per system): an unfinished
@@ -2390,22 +2313,6 @@ __global__ __launch_bounds__(256) void k_batch_fill(const int *row_off, const in
         const int o = act_off[s];
         for (int k = threadIdx.x; k < n; k += 256) list[o + k] = r0 + k;
     }
-}
-
-__global__ __launch_bounds__(256) void k_seg_sum(const double *x, const int *off, const int *done,
-                                                 double *out) {
-    __shared__ double part[256];
-    const int s = blockIdx.x;
-    if (done && done[s]) return;
-    double acc = 0.0;
-    for (int k = off[s] + (int) threadIdx.x; k < off[s + 1]; k += 256) acc += x[k];
-    part[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int) threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[s] = part[0];
 }
 
 // Per-system min of lo and max of hi (the max starting at DBL_MIN, as bml's
@@ -3153,12 +3060,43 @@ int win_pack(int N, int M, const void *Xv, const int *Xi, const int *Xn, int wbi
     return report("k_win_pack");
 }
 
+// The end of a product: its row records, and for x2 the traces.
+TailParams product_tail(const bmlhip_spgemm_args *a, const int4 *rowstat, const double *rowtr,
+                        int prec) {
+    TailParams tp{};
+    tp.N = a->N;
+    tp.MC = a->MC;
+    // kind 1 (AB) checks the distinct count against MC, as the reference does
+    // (the fused epilogue folds that check into the kept count it records)
+    tp.what = (a->kind == 1 && !a->fuse ? BMLHIP_RS_OVF_DIST : BMLHIP_RS_OVF_KEPT) |
+              BMLHIP_RS_STORED | BMLHIP_RS_PROF;
+    tp.prof = prec;
+    tp.skip = a->d_skip;
+    tp.rowstat = rowstat;
+    tp.st = bmlhip_status_dev();
+    tp.host = bmlhip_host_dev();
+    if (a->sp2) tp.sp2 = *a->sp2;
+    if (a->kind == 0) {
+        tp.nsum = 2;
+        tp.x[0] = rowtr;
+        tp.x[1] = rowtr + a->N;
+        tp.out[0] = a->batch ? a->batch->d_trx : &tp.st->scalars[0];
+        tp.out[1] = a->batch ? a->batch->d_trx2 : &tp.st->scalars[1];
+        if (a->batch) {
+            tp.nsys = a->batch->nsys;
+            tp.row_off = a->batch->d_row_off;
+            tp.done = a->batch->d_done;
+        }
+    }
+    return tp;
+}
+
 // X^2 on the window engine (a->d_Av == a->d_Bv): pack, rows, mirror (sym),
 // row records and traces, as spgemm_typed's other engines.
 template <typename T>
 int spgemm_win_typed(const bmlhip_spgemm_args *a) {
     hipStream_t s = (hipStream_t) bmlhip_stream();
-    int rc = bmlhip_status_reset();
+    int rc = bmlhip_status_ready();
     if (rc) return rc;
     WinParams wp;
     memset(&wp, 0, sizeof wp);
@@ -3215,24 +3153,9 @@ int spgemm_win_typed(const bmlhip_spgemm_args *a) {
         if ((rc = report("k_sym_mirror"))) return rc;
     }
     if (a->N > 0) bmlhip_prof_mark_end();
-    hipLaunchKernelGGL(k_reduce_rowstat, dim3(rowstat_blocks(a->N)), dim3(256), 0, s,
-                       (const int4 *) wp.rowstat, a->N, a->MC,
-                       BMLHIP_RS_OVF_KEPT | BMLHIP_RS_STORED | BMLHIP_RS_PROF |
-                           (rows > 1 ? BMLHIP_RS_OWN_STREAM : 0),
-                       (int) PrecOf<T>::value, a->d_skip, bmlhip_status_dev());
-    if ((rc = report("k_reduce_rowstat"))) return rc;
-    bmlhip_status *st = bmlhip_status_dev();
-    if (a->batch) {
-        const bmlhip_batch *b = a->batch;
-        hipLaunchKernelGGL(k_seg_sum, dim3(b->nsys), dim3(256), 0, s, wp.rowtr, b->d_row_off,
-                           b->d_done, b->d_trx);
-        hipLaunchKernelGGL(k_seg_sum, dim3(b->nsys), dim3(256), 0, s, wp.rowtr + a->N,
-                           b->d_row_off, b->d_done, b->d_trx2);
-        return report("k_seg_sum");
-    }
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, wp.rowtr, a->N, &st->scalars[0]);
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, wp.rowtr + a->N, a->N, &st->scalars[1]);
-    return report("k_sum");
+    TailParams tp = product_tail(a, wp.rowstat, wp.rowtr, (int) PrecOf<T>::value);
+    if (rows > 1) tp.what |= BMLHIP_RS_OWN_STREAM;
+    return launch_tail(tp, s);
 }
 
 // One fused SP2 iteration on the window engine (symmetric X, in place).
@@ -3241,7 +3164,7 @@ int sp2_window_typed(int N, int M, void *Xv, int *Xi, int *Xn, double thr, int w
                      int wrows, bmlhip_sp2_state *d_state, double nocc, double tol,
                      double *d_hist, int maxit) {
     hipStream_t s = (hipStream_t) bmlhip_stream();
-    int rc = bmlhip_status_reset();
+    int rc = bmlhip_status_ready();
     if (rc) return rc;
     bmlhip_status *st = bmlhip_status_dev();
     const int *skip = &d_state->done;
@@ -3258,10 +3181,24 @@ int sp2_window_typed(int N, int M, void *Xv, int *Xi, int *Xn, double thr, int w
         return rc;
     wp.streamed = rows > 1 ? (unsigned long long *) &st->prof_streamed[PrecOf<T>::value] : nullptr;
     // the branch needs tr X and tr X^2 before the product
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, rowtr, N, &st->scalars[0]);
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, rowtr + N, N, &st->scalars[1]);
-    if ((rc = report("k_sum"))) return rc;
-    if ((rc = bmlhip_sp2_decide(d_state, nocc, d_hist, maxit))) return rc;
+    TailParams tp{};
+    tp.N = N;
+    tp.MC = M;
+    tp.skip = skip;
+    tp.nsum = 2;
+    tp.x[0] = rowtr;
+    tp.x[1] = rowtr + N;
+    tp.out[0] = &st->scalars[0];
+    tp.out[1] = &st->scalars[1];
+    tp.st = st;
+    tp.host = bmlhip_host_dev();
+    tp.sp2.op = BMLHIP_TAIL_DECIDE;
+    tp.sp2.state = d_state;
+    tp.sp2.nocc = nocc;
+    tp.sp2.tol = tol;
+    tp.sp2.hist = d_hist;
+    tp.sp2.maxit = maxit;
+    if ((rc = launch_tail(tp, s))) return rc;
     wp.MC = M;
     wp.Cv = Xv;
     wp.Ci = Xi;
@@ -3289,14 +3226,16 @@ int sp2_window_typed(int N, int M, void *Xv, int *Xi, int *Xn, double thr, int w
         if ((rc = report("k_sym_mirror"))) return rc;
         bmlhip_prof_mark_end();
     }
-    hipLaunchKernelGGL(k_reduce_rowstat, dim3(rowstat_blocks(N)), dim3(256), 0, s,
-                       (const int4 *) rowstat, N, M,
-                       BMLHIP_RS_OVF_KEPT | BMLHIP_RS_STORED | BMLHIP_RS_PROF |
-                           (rows > 1 ? BMLHIP_RS_OWN_STREAM : 0),
-                       (int) PrecOf<T>::value, skip, st);
-    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, rownorm, N, &st->scalars[2]);
-    if ((rc = report("k_sum"))) return rc;
-    return bmlhip_sp2_check(d_state, tol, d_hist, maxit, 1);
+    tp.what = BMLHIP_RS_OVF_KEPT | BMLHIP_RS_STORED | BMLHIP_RS_PROF |
+              (rows > 1 ? BMLHIP_RS_OWN_STREAM : 0);
+    tp.prof = (int) PrecOf<T>::value;
+    tp.rowstat = rowstat;
+    tp.nsum = 1;
+    tp.x[0] = rownorm;
+    tp.out[0] = &st->scalars[2];
+    tp.sp2.op = BMLHIP_TAIL_CHECK;
+    tp.sp2.touched = 1;
+    return launch_tail(tp, s);
 }
 
 template <typename T>
@@ -3394,7 +3333,7 @@ int spgemm_typed(const bmlhip_spgemm_args *a) {
     long long tsize = ((long long) a->table + 7) & ~7ll;
     if (tsize < 64) tsize = 64;
     if (tsize > 65528) tsize = 65528;
-    int rc = bmlhip_status_reset();
+    int rc = bmlhip_status_ready();
     if (rc) return rc;
     const unsigned ts = (unsigned) tsize;
     const bool sym = a->sym && a->kind == 0 && a->engine == BMLHIP_ROW_UNORDERED && a->group == 64;
@@ -3449,44 +3388,28 @@ int spgemm_typed(const bmlhip_spgemm_args *a) {
         return fail_msg(2, "group %d not one of 8/16/32/64", a->group);
     }
     if (rc) return rc;
-    hipLaunchKernelGGL(k_spgemm_global<T>, dim3(gblocks), dim3(64), 0, s, p, (unsigned) gsize, gtab,
-                       cursor);
-    if ((rc = report("k_spgemm_global"))) return rc;
+    // (the direct kernel on columns that are their own slots has room for
+    // every row: see pick_direct)
+    if (!(direct && a->wbits == BMLHIP_DIR_DENSE)) {
+        hipLaunchKernelGGL(k_spgemm_global<T>, dim3(gblocks), dim3(64), 0, s, p, (unsigned) gsize,
+                           gtab, cursor);
+        if ((rc = report("k_spgemm_global"))) return rc;
+    }
     if (sym && a->N > 0) {
         hipLaunchKernelGGL(k_sym_mirror<T>, dim3((a->N + 3) / 4), dim3(256), 0, s, p, fill);
         hipLaunchKernelGGL(k_sym_finish, dim3((a->N + 255) / 256), dim3(256), 0, s, p, fill);
         bmlhip_prof_mark_end();
         if ((rc = report("k_sym_mirror"))) return rc;
     }
-    // kind 1 (AB) checks the distinct count against MC, as the reference does
-    // (the fused epilogue folds that check into the kept count it records)
-    hipLaunchKernelGGL(k_reduce_rowstat, dim3(rowstat_blocks(a->N)), dim3(256), 0, s,
-                       (const int4 *) p.rowstat, a->N, a->MC,
-                       (a->kind == 1 && !a->fuse ? BMLHIP_RS_OVF_DIST : BMLHIP_RS_OVF_KEPT) |
-                           BMLHIP_RS_STORED | BMLHIP_RS_PROF,
-                       (int) PrecOf<T>::value, p.skip, p.st);
-    if ((rc = report("k_reduce_rowstat"))) return rc;
-    if (a->kind == 0 && a->batch) {
-        const bmlhip_batch *b = a->batch;
-        hipLaunchKernelGGL(k_seg_sum, dim3(b->nsys), dim3(256), 0, s, p.rowtr, b->d_row_off,
-                           b->d_done, b->d_trx);
-        hipLaunchKernelGGL(k_seg_sum, dim3(b->nsys), dim3(256), 0, s, p.rowtr + a->N,
-                           b->d_row_off, b->d_done, b->d_trx2);
-        if ((rc = report("k_seg_sum"))) return rc;
-    } else if (a->kind == 0) {
-        hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, p.rowtr, a->N, &p.st->scalars[0]);
-        hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, p.rowtr + a->N, a->N,
-                           &p.st->scalars[1]);
-        if ((rc = report("k_sum"))) return rc;
-    }
-    return 0;
+    return launch_tail(product_tail(a, p.rowstat, p.rowtr, (int) PrecOf<T>::value), s);
 }
 
 template <typename T>
 int add_typed(int N, int MA, void *Av, int *Ai, int *An, int MB, const void *Bv, const int *Bi,
               const int *Bn, double alpha, double beta, double thr, int mode,
               const double *abdev = nullptr, const int *skip = nullptr,
-              const bmlhip_batch *batch = nullptr, double *rownorm = nullptr) {
+              const bmlhip_batch *batch = nullptr, double *rownorm = nullptr,
+              const bmlhip_sp2_tail *sp2 = nullptr) {
     hipStream_t s = (hipStream_t) bmlhip_stream();
     AddParams p{};
     p.N = N;
@@ -3513,7 +3436,7 @@ int add_typed(int N, int MA, void *Av, int *Ai, int *An, int MB, const void *Bv,
     p.rownorm = rownorm ? rownorm : (double *) bmlhip_scratch(0, sizeof(double) * (size_t) (N + 1));
     p.rowstat = (int4 *) bmlhip_scratch(BMLHIP_ROWSTAT_SLOT, sizeof(int4) * (size_t) (N + 1));
     if (!p.rownorm || !p.rowstat) return 4;
-    int rc = bmlhip_status_reset();
+    int rc = bmlhip_status_ready();
     if (rc) return rc;
     // a row's union has at most MA + MB columns: the LDS table keeps it at
     // most 4/5 full (multiple of 64 slots; first-touch list in 16 bits)
@@ -3534,20 +3457,27 @@ int add_typed(int N, int MA, void *Av, int *Ai, int *An, int MB, const void *Bv,
             hipLaunchKernelGGL(k_add_global<T>, dim3(blocks), dim3(64), 0, s, p, tbits, tabs);
             if ((rc = report("k_add_global"))) return rc;
         }
-        hipLaunchKernelGGL(k_reduce_rowstat, dim3(rowstat_blocks(N)), dim3(256), 0, s,
-                           (const int4 *) p.rowstat, N, MA,
-                           BMLHIP_RS_OVF_KEPT | BMLHIP_RS_STORED, 0, skip, p.st);
-        if ((rc = report("k_reduce_rowstat"))) return rc;
     }
-    if (mode && batch) {
-        hipLaunchKernelGGL(k_seg_sum, dim3(batch->nsys), dim3(256), 0, s, p.rownorm,
-                           batch->d_row_off, batch->d_done, batch->d_norm2);
-        if ((rc = report("k_seg_sum"))) return rc;
-    } else if (mode) {
-        hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, p.rownorm, N, &p.st->scalars[2]);
-        if ((rc = report("k_sum"))) return rc;
+    TailParams tp{};
+    tp.N = N;
+    tp.MC = MA;
+    tp.what = BMLHIP_RS_OVF_KEPT | BMLHIP_RS_STORED;
+    tp.skip = skip;
+    tp.rowstat = p.rowstat;
+    tp.st = p.st;
+    tp.host = bmlhip_host_dev();
+    if (sp2) tp.sp2 = *sp2;
+    if (mode) {
+        tp.nsum = 1;
+        tp.x[0] = p.rownorm;
+        tp.out[0] = batch ? batch->d_norm2 : &p.st->scalars[2];
+        if (batch) {
+            tp.nsys = batch->nsys;
+            tp.row_off = batch->d_row_off;
+            tp.done = batch->d_done;
+        }
     }
-    return 0;
+    return launch_tail(tp, s);
 }
 
 template <typename T>
@@ -3746,8 +3676,8 @@ int bmlhip_is_symmetric(int prec, int N, int M, const void *Av, const int *Ai, c
 
 int bmlhip_add_dev(int prec, int N, int MA, void *Av, int *Ai, int *An, int MB, const void *Bv,
                    const int *Bi, const int *Bn, const double *ab, double thr, int mode,
-                   const int *skip) {
-#define CALL(T) add_typed<T>(N, MA, Av, Ai, An, MB, Bv, Bi, Bn, 0.0, 0.0, thr, mode, ab, skip)
+                   const int *skip, const bmlhip_sp2_tail *sp2) {
+#define CALL(T) add_typed<T>(N, MA, Av, Ai, An, MB, Bv, Bi, Bn, 0.0, 0.0, thr, mode, ab, skip, nullptr, nullptr, sp2)
     DISPATCH(prec, CALL)
 #undef CALL
 }
@@ -3804,8 +3734,8 @@ int bmlhip_batch_queue(const bmlhip_batch *b, int N) {
 }
 
 int bmlhip_add_batch(int prec, int N, int MA, void *Av, int *Ai, int *An, int MB, const void *Bv,
-                     const int *Bi, const int *Bn, double thr, int mode, const bmlhip_batch *b) {
-#define CALL(T) add_typed<T>(N, MA, Av, Ai, An, MB, Bv, Bi, Bn, 0.0, 0.0, thr, mode, nullptr, nullptr, b, b->d_rownorm)
+                     const int *Bi, const int *Bn, double thr, int mode, const bmlhip_batch *b, const bmlhip_sp2_tail *sp2) {
+#define CALL(T) add_typed<T>(N, MA, Av, Ai, An, MB, Bv, Bi, Bn, 0.0, 0.0, thr, mode, nullptr, nullptr, b, b->d_rownorm, sp2)
     DISPATCH(prec, CALL)
 #undef CALL
 }

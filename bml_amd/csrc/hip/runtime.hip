@@ -18,6 +18,9 @@ struct Runtime {
     int device = -1;
     hipStream_t stream = nullptr;
     bmlhip_status *status = nullptr;
+    bmlhip_host *host = nullptr;  // pinned
+    bool clear = false;      // the status block's per-operation fields are reset
+    bool published = false;  // host->status is the last operation's
     void *scratch[BMLHIP_SCRATCH_SLOTS] = {};
     size_t scratch_bytes[BMLHIP_SCRATCH_SLOTS] = {};
     char msg[512] = {0};
@@ -50,6 +53,7 @@ __global__ void k_status_reset(bmlhip_status *st, int clear_errors) {
         if (clear_errors) {
             st->m_overflow_rows = 0;
             st->first_m_overflow = INT_MAX;
+            st->tail_done = 0;
         }
         st->table_overflow_rows = 0;
         st->max_nnz = 0;
@@ -58,6 +62,13 @@ __global__ void k_status_reset(bmlhip_status *st, int clear_errors) {
         st->total_nnz = 0;
         for (int k = 0; k < 4; k++) st->scalars[k] = 0.0;
     }
+}
+
+// the status block as it is, to the host
+__global__ void k_publish(const bmlhip_status *st, bmlhip_host *host) {
+    const int words = (int) (sizeof(bmlhip_status) / sizeof(int));
+    for (int k = threadIdx.x; k < words; k += 64)
+        ((int *) &host->status)[k] = ((const int *) st)[k];
 }
 
 #define CHECK(call)                                   \
@@ -88,6 +99,9 @@ int bmlhip_init(int device) {
     }
     CHECK(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
     CHECK(hipMalloc((void **) &g.status, sizeof(bmlhip_status)));
+    CHECK(hipHostMalloc((void **) &g.host, sizeof(bmlhip_host), hipHostMallocDefault));
+    memset(g.host, 0, sizeof(bmlhip_host));
+    g.clear = g.published = false;
     hipLaunchKernelGGL(k_status_reset, dim3(1), dim3(64), 0, g.stream, g.status, 1);
     CHECK(hipGetLastError());
     CHECK(hipStreamSynchronize(g.stream));
@@ -104,6 +118,8 @@ void bmlhip_shutdown(void) {
         g.scratch_bytes[s] = 0;
     }
     (void) hipFree(g.status);
+    (void) hipHostFree(g.host);
+    g.host = nullptr;
     (void) hipStreamDestroy(g.stream);
     g.status = nullptr;
     g.stream = nullptr;
@@ -234,13 +250,26 @@ void *bmlhip_scratch_zeroed(int slot, size_t bytes) {
 
 bmlhip_status *bmlhip_status_dev(void) { return g.status; }
 
+bmlhip_host *bmlhip_host_dev(void) { return g.host; }
+
+void bmlhip_status_published(void) { g.clear = g.published = true; }
+
+int bmlhip_status_ready(void) {
+    if (g.clear) return 0;
+    const int rc = bmlhip_status_reset();
+    g.clear = rc == 0;
+    return rc;
+}
+
 int bmlhip_status_reset(void) {
+    g.clear = g.published = false;
     hipLaunchKernelGGL(k_status_reset, dim3(1), dim3(64), 0, g.stream, g.status, 0);
     CHECK(hipGetLastError());
     return 0;
 }
 
 int bmlhip_status_clear_errors(void) {
+    g.clear = g.published = false;
     hipLaunchKernelGGL(k_status_reset, dim3(1), dim3(64), 0, g.stream, g.status, 1);
     CHECK(hipGetLastError());
     return 0;
@@ -259,6 +288,7 @@ __global__ void k_prof_reset(bmlhip_status *st) {
 }
 
 int bmlhip_prof_begin(void) {
+    g.published = false;
     hipLaunchKernelGGL(k_prof_reset, dim3(1), dim3(64), 0, g.stream, g.status);
     CHECK(hipGetLastError());
     g.profiling = 1;
@@ -329,9 +359,27 @@ void bmlhip_graph_destroy(void *exec) {
 }
 
 int bmlhip_status_fetch(bmlhip_status *h) {
-    CHECK(hipMemcpyAsync(h, g.status, sizeof *h, hipMemcpyDeviceToHost, g.stream));
+    if (!g.published) {
+        hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, g.stream, g.status, g.host);
+        CHECK(hipGetLastError());
+    }
     CHECK(hipStreamSynchronize(g.stream));
     CHECK(hipGetLastError());
+    *h = g.host->status;
+    return 0;
+}
+
+int bmlhip_sp2_state_fetch(bmlhip_sp2_state *st) {
+    CHECK(hipStreamSynchronize(g.stream));
+    *st = g.host->state;
+    return 0;
+}
+
+int bmlhip_sp2_stats_fetch(int stats[2], int *alldone) {
+    CHECK(hipStreamSynchronize(g.stream));
+    stats[0] = g.host->stats[0];
+    stats[1] = g.host->stats[1];
+    *alldone = g.host->alldone;
     return 0;
 }
 

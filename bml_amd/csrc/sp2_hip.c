@@ -167,12 +167,23 @@ static int sp2_iteration(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpack_hip_t *
     a.d_Cv = X2->value;
     a.d_Ci = X2->index;
     a.d_Cn = X2->nnz;
-    return bmlh_ok(bmlhip_spgemm(&a), what) &&
-           bmlh_ok(bmlhip_sp2_decide(d_state, nocc, d_hist, o->maxit), what) &&
-           bmlh_ok(bmlhip_add_dev(X->matrix_precision, X->N, X->M, X->value, X->index, X->nnz,
+    /* the branch and the convergence test are taken where the product's
+     * traces and the update's norm are complete */
+    bmlhip_sp2_tail t;
+    memset(&t, 0, sizeof t);
+    t.op = BMLHIP_TAIL_DECIDE;
+    t.state = d_state;
+    t.nocc = nocc;
+    t.tol = o->tol;
+    t.hist = d_hist;
+    t.maxit = o->maxit;
+    a.sp2 = &t;
+    if (!bmlh_ok(bmlhip_spgemm(&a), what))
+        return 0;
+    t.op = BMLHIP_TAIL_CHECK;
+    return bmlh_ok(bmlhip_add_dev(X->matrix_precision, X->N, X->M, X->value, X->index, X->nnz,
                                   X2->M, X2->value, X2->index, X2->nnz, d_state->ab,
-                                  o->threshold, 2, &d_state->done), what) &&
-           bmlh_ok(bmlhip_sp2_check(d_state, o->tol, d_hist, o->maxit, 0), what);
+                                  o->threshold, 2, &d_state->done, &t), what);
 }
 
 void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_hip_t *X,
@@ -297,7 +308,7 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
         }
         int last_single = single && it + 1 >= o.maxit - o.refine_iters;
         if ((it + 1) % o.poll == 0 || last_single || it + 1 == o.maxit) {
-            if (!bmlh_ok(bmlhip_d2h(&st, d_state, sizeof st), what))
+            if (!bmlh_ok(bmlhip_sp2_state_fetch(&st), what))
                 goto out;
             /* the tuner reads max_nnz; the totals are refreshed at the end */
             cur->aux->touched_hint = st.max_touched;
@@ -321,7 +332,7 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
             single = 0;
         }
     }
-    if (!bmlh_ok(bmlhip_d2h(&st, d_state, sizeof st), what))
+    if (!bmlh_ok(bmlhip_sp2_state_fetch(&st), what))
         goto out;
     if (single) {
         /* converged while still in single precision: hand back in X */
@@ -420,12 +431,13 @@ static int batch_alloc(batch_dev *d, int nsys, int N, const char *what)
     d->b.d_norm2 = d->norm2;
     d->b.d_rowtr = d->rowtr;
     d->b.d_rownorm = d->rownorm;
-    /* The work queue is on for the exact engine and off for the others
-     * (their batched iterations ran faster with one block per row: 147
-     * against 129 solves/s on the 512-system batch); BML_HIP_BATCH_QUEUE=1
-     * or 0 sets it either way. */
+    /* The work queue (BML_HIP_BATCH_QUEUE=1) lists the unfinished systems'
+     * rows for persistent hash and add kernels; off, every row has its place
+     * in a grid and rows of finished systems return at once, which ran
+     * faster on every engine (unordered: 147 against 129 solves/s on the
+     * 512-system batch) */
     const char *e = getenv("BML_HIP_BATCH_QUEUE");
-    const int queue = e ? atoi(e) != 0 : bml_hip_get_row_engine() == BML_HIP_ROW_ENGINE_EXACT;
+    const int queue = e && atoi(e) != 0;
     if (queue) {
         d->b.d_list = d->list;
         d->b.d_qinfo = d->qinfo;
@@ -463,13 +475,25 @@ static int batch_iteration(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpack_hip_t
     a.wrows = sh->wrows;
     a.sym = d->sym;
     a.batch = &d->b;
-    return bmlh_ok(bmlhip_batch_queue(&d->b, X->N), what) && bmlh_ok(bmlhip_spgemm(&a), what) &&
-           bmlh_ok(bmlhip_sp2_decide_batch(&d->b, d->nocc, d->branch, d->stats), what) &&
-           bmlh_ok(bmlhip_add_batch(X->matrix_precision, X->N, X->M, X->value, X->index, X->nnz,
+    bmlhip_sp2_tail t;
+    memset(&t, 0, sizeof t);
+    t.op = BMLHIP_TAIL_DECIDE_BATCH;
+    t.tol = o->tol;
+    t.maxit = o->maxit;
+    t.d_nocc = d->nocc;
+    t.ab = d->ab;
+    t.norm = d->norm;
+    t.branch = d->branch;
+    t.it = d->it;
+    t.stats = d->stats;
+    t.alldone = d->alldone;
+    a.sp2 = &t;
+    if (!bmlh_ok(bmlhip_batch_queue(&d->b, X->N), what) || !bmlh_ok(bmlhip_spgemm(&a), what))
+        return 0;
+    t.op = BMLHIP_TAIL_CHECK_BATCH;
+    return bmlh_ok(bmlhip_add_batch(X->matrix_precision, X->N, X->M, X->value, X->index, X->nnz,
                                     X2->M, X2->value, X2->index, X2->nnz, o->threshold, 2,
-                                    &d->b), what) &&
-           bmlh_ok(bmlhip_sp2_check_batch(&d->b, o->tol, o->maxit, d->it, d->norm, d->alldone,
-                                          d->stats), what);
+                                    &d->b, &t), what);
 }
 
 void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
@@ -604,7 +628,7 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
             span = hi - lo;
         lo += H[s]->N;
     }
-    int touched = 0, hint_max = 0, stats[2] = { 0, 0 }, alldone[2] = { 0, 0 };
+    int touched = 0, hint_max = 0, stats[2] = { 0, 0 }, alldone = 0;
     for (int it = 0; it < o.maxit; it++) {
         bml_matrix_ellpack_hip_t *cur = single ? Xs : Xc, *cur2 = single ? X2s : X2c;
         const int mx = cur->aux->stats_valid ? cur->aux->max_nnz : cur->M;
@@ -639,14 +663,13 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
         }
         const int last_single = single && it + 1 >= o.maxit - o.refine_iters;
         if ((it + 1) % o.poll == 0 || last_single || it + 1 == o.maxit) {
-            if (!bmlh_ok(bmlhip_d2h(alldone, d.alldone, sizeof alldone), what) ||
-                !bmlh_ok(bmlhip_d2h(stats, d.stats, sizeof stats), what))
+            if (!bmlh_ok(bmlhip_sp2_stats_fetch(stats, &alldone), what))
                 goto out;
             touched = stats[0];
             hint_max = mx;
             cur->aux->stats_valid = 1;
             cur->aux->max_nnz = stats[1];
-            if (alldone[0] >= nsys)
+            if (alldone >= nsys)
                 break;
         }
         if (last_single) {
