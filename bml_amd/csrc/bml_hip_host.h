@@ -18,6 +18,8 @@ struct bml_hip_aux {
     int touched_hint;      /* distinct columns per row seen the last time this
                               matrix was squared (0 = unknown) */
     int hint_max_nnz;      /* its longest row at that time */
+    int temp;              /* a call's temporary: arrays from bmlhip_temp_malloc
+                              (an ellblock's bsize is another matrix's) */
     int len_hint;          /* stats not valid: about the longest row (0 = unknown;
                               launch shapes only) */
 };
@@ -42,10 +44,13 @@ int bmlh_sync_mode(void);
 size_t bmlh_elem_size(int precision);
 /* block-product engine for products of A (BML_HIP_BLOCK_ENGINE_*, resolved) */
 int bmlh_block_engine_for(const bml_matrix_ellblock_hip_t *A);
-/* An ELLBLOCK work matrix with undefined tile values (indices and counts
- * zero), for drivers that write every tile before reading it. */
-bml_matrix_ellblock_hip_t *bmlh_block_matrix_ellblock_work(int precision, int NB, int MB, int M,
-                                                           const int *bsize, int distrib_mode);
+/* Temporaries of a call: an ELLBLOCK matrix of A's block structure with
+ * undefined blocks (counts zero), for drivers that write every block before
+ * they read it, and an ELLPACK matrix with undefined rows (counts zero).
+ * Freed by bml_deallocate_*. */
+bml_matrix_ellblock_hip_t *bmlh_temp_matrix_ellblock(const bml_matrix_ellblock_hip_t *A,
+                                                     int precision, int MB);
+bml_matrix_ellpack_hip_t *bmlh_temp_matrix_ellpack(int precision, int N, int M, int distrib_mode);
 /* the engine set by bml_hip_set_block_engine (BML_HIP_BLOCK_ENGINE_*) */
 int bmlh_block_engine_setting(void);
 /* the real scalar s as one element of precision prec, into buf (16 bytes) */
@@ -53,6 +58,8 @@ void bmlh_put_scalar(int prec, double s, void *buf);
 struct bml_hip_aux *bmlh_aux_new(void);
 /* the row statistics no longer hold: rows may have grown by `more` entries */
 void bmlh_stats_stale(struct bml_hip_aux *aux, int more);
+/* dst's rows are copies of src's */
+void bmlh_copy_stats(struct bml_hip_aux *dst, const struct bml_hip_aux *src);
 void bmlh_set_stats(struct bml_hip_aux *aux, const bmlhip_status *st);
 /* The row-major dense N x N host array (malloc'd) of an ellpack_hip or
  * ellblock_hip matrix A, its elements cast to precision; N into *N_out. */

@@ -148,6 +148,13 @@ void bmlh_set_stats(struct bml_hip_aux *aux, const bmlhip_status *st)
     }
 }
 
+void bmlh_copy_stats(struct bml_hip_aux *dst, const struct bml_hip_aux *src)
+{
+    const int temp = dst->temp;
+    *dst = *src;
+    dst->temp = temp;
+}
+
 void bmlh_stats_stale(struct bml_hip_aux *aux, int more)
 {
     if (aux->stats_valid)

@@ -68,6 +68,10 @@ void *bmlhip_noalloc_workspace(size_t *bytes);
 void bmlhip_set_errmsg(const char *msg);
 int bmlhip_malloc(void **d_ptr, size_t bytes);
 void bmlhip_free(void *d_ptr);
+/* device memory of a call's temporaries: kept and handed out again in stream
+ * order (bounded; either free takes either kind) */
+int bmlhip_temp_malloc(void **d_ptr, size_t bytes);
+void bmlhip_temp_free(void *d_ptr);
 int bmlhip_h2d(void *d_dst, const void *src, size_t bytes);
 int bmlhip_d2h(void *dst, const void *d_src, size_t bytes);
 int bmlhip_d2d(void *d_dst, const void *d_src, size_t bytes);
@@ -158,7 +162,7 @@ typedef struct bmlhip_batch {
      * in order, rebuilt on the device before each product; the row kernels
      * then run persistent, taking rows from it with an atomic cursor */
     int *d_list;           /* [N] */
-    int *d_qinfo;          /* [4]: rows listed, product cursor, add cursor, systems left */
+    int *d_qinfo;          /* [4]: rows listed, product cursor, unused, systems left */
     int *d_act_off;        /* [nsys + 1] first list position of each system */
 } bmlhip_batch;
 

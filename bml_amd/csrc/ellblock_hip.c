@@ -166,7 +166,8 @@ static void eb_finish_into(const char *what, bml_matrix_ellblock_hip_t *out)
 /* ---- allocation ------------------------------------------------------------ */
 
 static bml_matrix_ellblock_hip_t *eb_alloc(int precision, int NB, int MB, int M,
-                                           const int *bsize, int distrib_mode, int zero_values)
+                                           const int *bsize, int distrib_mode,
+                                           const bml_matrix_ellblock_hip_t *like)
 {
     const char *what = "bml_block_matrix_ellblock_hip";
     if (bmlh_ready())
@@ -213,6 +214,20 @@ static bml_matrix_ellblock_hip_t *eb_alloc(int precision, int NB, int MB, int M,
     }
     memcpy(A->bsize_host, bsize, sizeof(int) * (size_t) NB);
     const size_t slots = (size_t) NB * MB;
+    if (like) {
+        /* a temporary with the structure of `like` */
+        A->aux->temp = 1;
+        A->bsize = like->bsize;
+        if (!bmlh_ok(bmlhip_temp_malloc(&A->value, slots * tile_bytes(A)), what) ||
+            !bmlh_ok(bmlhip_temp_malloc((void **) &A->indexb, slots * sizeof(int)), what) ||
+            !bmlh_ok(bmlhip_temp_malloc((void **) &A->nnzb, (size_t) NB * sizeof(int)), what)) {
+            bml_deallocate_ellblock_hip(A);
+            return NULL;
+        }
+        bmlhip_zero(A->nnzb, (size_t) NB * sizeof(int));
+        A->aux->stats_valid = 1;
+        return A;
+    }
     if (!bmlh_ok(bmlhip_malloc(&A->value, slots * tile_bytes(A)), what) ||
         !bmlh_ok(bmlhip_malloc((void **) &A->indexb, slots * sizeof(int)), what) ||
         !bmlh_ok(bmlhip_malloc((void **) &A->nnzb, (size_t) NB * sizeof(int)), what) ||
@@ -221,8 +236,7 @@ static bml_matrix_ellblock_hip_t *eb_alloc(int precision, int NB, int MB, int M,
         bml_deallocate_ellblock_hip(A);
         return NULL;
     }
-    if (zero_values)
-        bmlhip_zero(A->value, slots * tile_bytes(A));
+    bmlhip_zero(A->value, slots * tile_bytes(A));
     bmlhip_zero(A->indexb, slots * sizeof(int));
     bmlhip_zero(A->nnzb, (size_t) NB * sizeof(int));
     A->aux->stats_valid = 1;
@@ -234,16 +248,13 @@ static bml_matrix_ellblock_hip_t *eb_alloc(int precision, int NB, int MB, int M,
 bml_matrix_ellblock_hip_t *bml_block_matrix_ellblock_hip(int precision, int NB, int MB, int M,
                                                          const int *bsize, int distrib_mode)
 {
-    return eb_alloc(precision, NB, MB, M, bsize, distrib_mode, 1);
+    return eb_alloc(precision, NB, MB, M, bsize, distrib_mode, NULL);
 }
 
-/* A work matrix whose tile values start undefined (block counts zero): for
- * drivers that write every tile they later read, so the NB*MB tiles of a
- * wide matrix are not cleared on every call */
-bml_matrix_ellblock_hip_t *bmlh_block_matrix_ellblock_work(int precision, int NB, int MB, int M,
-                                                           const int *bsize, int distrib_mode)
+bml_matrix_ellblock_hip_t *bmlh_temp_matrix_ellblock(const bml_matrix_ellblock_hip_t *A,
+                                                     int precision, int MB)
 {
-    return eb_alloc(precision, NB, MB, M, bsize, distrib_mode, 0);
+    return eb_alloc(precision, A->NB, MB, A->M, A->bsize_host, A->distribution_mode, A);
 }
 
 bml_matrix_ellblock_hip_t *bml_zero_matrix_ellblock_hip(int precision, int N, int M,
@@ -259,10 +270,16 @@ void bml_deallocate_ellblock_hip(bml_matrix_ellblock_hip_t *A)
 {
     if (!A)
         return;
-    bmlhip_free(A->value);
-    bmlhip_free(A->indexb);
-    bmlhip_free(A->nnzb);
-    bmlhip_free(A->bsize);
+    if (A->aux && A->aux->temp) {
+        bmlhip_temp_free(A->value);
+        bmlhip_temp_free(A->indexb);
+        bmlhip_temp_free(A->nnzb);
+    } else {
+        bmlhip_free(A->value);
+        bmlhip_free(A->indexb);
+        bmlhip_free(A->nnzb);
+        bmlhip_free(A->bsize);
+    }
     free(A->bsize_host);
     free(A->aux);
     free(A);
@@ -286,7 +303,7 @@ void bml_copy_ellblock_hip(const bml_matrix_ellblock_hip_t *A, bml_matrix_ellblo
     if (!bmlh_ok(bmlhip_eb_copy(A->matrix_precision, A->NB, A->bt, A->MB, A->value, A->indexb,
                                 A->nnzb, B->MB, B->value, B->indexb, B->nnzb), what))
         return;
-    *B->aux = *A->aux;
+    bmlh_copy_stats(B->aux, A->aux);
     bmlhip_status st;
     bmlh_finish(what, &st);
 }
@@ -600,8 +617,7 @@ void bml_multiply_ellblock_hip(bml_matrix_ellblock_hip_t *A, bml_matrix_ellblock
         return;
     }
     /* product into a temporary with C's block slots, then C <- beta*C + alpha*T */
-    bml_matrix_ellblock_hip_t *T = bml_block_matrix_ellblock_hip(
-        A->matrix_precision, A->NB, C->MB, C->M, A->bsize_host, A->distribution_mode);
+    bml_matrix_ellblock_hip_t *T = bmlh_temp_matrix_ellblock(A, A->matrix_precision, C->MB);
     if (!T)
         return;
     if (A == B)

@@ -60,7 +60,7 @@ static int max_nnz_of(const bml_matrix_ellpack_hip_t *A)
     return A->aux->len_hint > 0 && A->aux->len_hint < A->M ? A->aux->len_hint : A->M;
 }
 
-static bml_matrix_ellpack_hip_t *alloc_ell(int prec, int N, int M, int mode, int zero,
+static bml_matrix_ellpack_hip_t *alloc_ell(int prec, int N, int M, int mode, int zero, int temp,
                                            const char *what)
 {
     if (bmlh_ready())
@@ -92,9 +92,11 @@ static bml_matrix_ellpack_hip_t *alloc_ell(int prec, int N, int M, int mode, int
     A->M = M;
     A->aux = bmlh_aux_new();
     size_t nm = (size_t) N * (size_t) M;
-    if (!bmlh_ok(bmlhip_malloc(&A->value, nm * es), what) ||
-        !bmlh_ok(bmlhip_malloc((void **) &A->index, nm * sizeof(int)), what) ||
-        !bmlh_ok(bmlhip_malloc((void **) &A->nnz, (size_t) N * sizeof(int)), what)) {
+    int (*get)(void **, size_t) = temp ? bmlhip_temp_malloc : bmlhip_malloc;
+    A->aux->temp = temp;
+    if (!bmlh_ok(get(&A->value, nm * es), what) ||
+        !bmlh_ok(get((void **) &A->index, nm * sizeof(int)), what) ||
+        !bmlh_ok(get((void **) &A->nnz, (size_t) N * sizeof(int)), what)) {
         bml_deallocate_ellpack_hip(A);
         return NULL;
     }
@@ -121,20 +123,25 @@ static void finish_into(const char *what, bml_matrix_ellpack_hip_t *out)
 bml_matrix_ellpack_hip_t *bml_zero_matrix_ellpack_hip(int precision, int N, int M,
                                                       int distrib_mode)
 {
-    return alloc_ell(precision, N, M, distrib_mode, 1, "bml_zero_matrix_ellpack_hip");
+    return alloc_ell(precision, N, M, distrib_mode, 1, 0, "bml_zero_matrix_ellpack_hip");
 }
 
 bml_matrix_ellpack_hip_t *bml_noinit_matrix_ellpack_hip(int precision, int N, int M,
                                                         int distrib_mode)
 {
-    return alloc_ell(precision, N, M, distrib_mode, 0, "bml_noinit_matrix_ellpack_hip");
+    return alloc_ell(precision, N, M, distrib_mode, 0, 0, "bml_noinit_matrix_ellpack_hip");
+}
+
+bml_matrix_ellpack_hip_t *bmlh_temp_matrix_ellpack(int precision, int N, int M, int distrib_mode)
+{
+    return alloc_ell(precision, N, M, distrib_mode, 0, 1, "bml_hip temporary");
 }
 
 bml_matrix_ellpack_hip_t *bml_identity_matrix_ellpack_hip(int precision, int N, int M,
                                                           int distrib_mode)
 {
     bml_matrix_ellpack_hip_t *A =
-        alloc_ell(precision, N, M, distrib_mode, 1, "bml_identity_matrix_ellpack_hip");
+        alloc_ell(precision, N, M, distrib_mode, 1, 0, "bml_identity_matrix_ellpack_hip");
     if (!A)
         return NULL;
     if (!bmlh_ok(bmlhip_identity(precision, N, M, A->value, A->index, A->nnz),
@@ -150,9 +157,10 @@ void bml_deallocate_ellpack_hip(bml_matrix_ellpack_hip_t *A)
 {
     if (!A)
         return;
-    bmlhip_free(A->value);
-    bmlhip_free(A->index);
-    bmlhip_free(A->nnz);
+    void (*put)(void *) = A->aux && A->aux->temp ? bmlhip_temp_free : bmlhip_free;
+    put(A->value);
+    put(A->index);
+    put(A->nnz);
     free(A->aux);
     free(A);
 }
@@ -181,7 +189,7 @@ void bml_copy_ellpack_hip(const bml_matrix_ellpack_hip_t *A, bml_matrix_ellpack_
             !bmlh_ok(bmlhip_d2d(B->index, A->index, nm * sizeof(int)), what) ||
             !bmlh_ok(bmlhip_d2d(B->nnz, A->nnz, (size_t) A->N * sizeof(int)), what))
             return;
-        *B->aux = *A->aux;
+        bmlh_copy_stats(B->aux, A->aux);
         bmlhip_status st;
         bmlh_finish(what, &st);
         return;
@@ -189,7 +197,7 @@ void bml_copy_ellpack_hip(const bml_matrix_ellpack_hip_t *A, bml_matrix_ellpack_
     if (!bmlh_ok(bmlhip_copy_rows(A->matrix_precision, A->N, A->M, A->value, A->index, A->nnz,
                                   B->M, B->value, B->index, B->nnz), what))
         return;
-    *B->aux = *A->aux;
+    bmlh_copy_stats(B->aux, A->aux);
     bmlhip_status st;
     bmlh_finish(what, &st);
 }
@@ -667,7 +675,7 @@ void bml_multiply_ellpack_hip(bml_matrix_ellpack_hip_t *A, bml_matrix_ellpack_hi
     /* C is A or B: the product into a temporary of C's shape, then
      * C <- beta*C + alpha*T */
     bml_matrix_ellpack_hip_t *T =
-        bml_noinit_matrix_ellpack_hip(A->matrix_precision, A->N, C->M, A->distribution_mode);
+        bmlh_temp_matrix_ellpack(A->matrix_precision, A->N, C->M, A->distribution_mode);
     if (!T)
         return;
     if (A == B)

@@ -73,7 +73,7 @@ static int measure_sp2(const bmlh_spgemm_shape *sh, void *ctx, double *ms)
 {
     sp2_tune_ctx *c = ctx;
     bml_matrix_ellpack_hip_t *X = c->X;
-    if (!*c->X2p && !(*c->X2p = bml_noinit_matrix_ellpack_hip(X->matrix_precision, X->N, X->M,
+    if (!*c->X2p && !(*c->X2p = bmlh_temp_matrix_ellpack(X->matrix_precision, X->N, X->M,
                                                               X->distribution_mode)))
         return 1;
     bml_matrix_ellpack_hip_t *X2 = *c->X2p;
@@ -159,7 +159,7 @@ static int sp2_iteration(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpack_hip_t *
                                               sh.waves, sh.wrows, d_state, nocc, o->tol, d_hist,
                                               o->maxit),
                        what);
-    if (!*X2p && !(*X2p = bml_noinit_matrix_ellpack_hip(X->matrix_precision, X->N, X->M,
+    if (!*X2p && !(*X2p = bmlh_temp_matrix_ellpack(X->matrix_precision, X->N, X->M,
                                                         X->distribution_mode)))
         return 0;
     bml_matrix_ellpack_hip_t *X2 = *X2p;
@@ -250,22 +250,22 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
     const bml_matrix_ellpack_hip_t *gcur = NULL;
     bmlh_spgemm_shape gshape;
     memset(&gshape, 0, sizeof gshape);
-    if (!bmlh_ok(bmlhip_malloc((void **) &d_state, sizeof(bmlhip_sp2_state)), what) ||
-        !bmlh_ok(bmlhip_malloc((void **) &d_hist, sizeof(double) * 4 * (size_t) o.maxit), what))
+    if (!bmlh_ok(bmlhip_temp_malloc((void **) &d_state, sizeof(bmlhip_sp2_state)), what) ||
+        !bmlh_ok(bmlhip_temp_malloc((void **) &d_hist, sizeof(double) * 4 * (size_t) o.maxit), what))
         goto out;
     bmlhip_zero(d_state, sizeof(bmlhip_sp2_state));
     bmlhip_zero(d_hist, sizeof(double) * 4 * (size_t) o.maxit);
 
     int single = 0;
     if (o.mixed && o.maxit > o.refine_iters) {
-        Xs = bml_noinit_matrix_ellpack_hip(sprec, N, M, X->distribution_mode);
+        Xs = bmlh_temp_matrix_ellpack(sprec, N, M, X->distribution_mode);
         if (!Xs)
             goto out;
         if (!bmlh_ok(bmlhip_convert(prec, sprec, (size_t) N * M, X->value, Xs->value), what) ||
             !bmlh_ok(bmlhip_d2d(Xs->index, X->index, (size_t) N * M * sizeof(int)), what) ||
             !bmlh_ok(bmlhip_d2d(Xs->nnz, X->nnz, (size_t) N * sizeof(int)), what))
             goto out;
-        *Xs->aux = *X->aux;
+        bmlh_copy_stats(Xs->aux, X->aux);
         single = 1;
     }
 
@@ -328,7 +328,7 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
                 !bmlh_ok(bmlhip_d2d(X->index, Xs->index, (size_t) N * M * sizeof(int)), what) ||
                 !bmlh_ok(bmlhip_d2d(X->nnz, Xs->nnz, (size_t) N * sizeof(int)), what))
                 goto out;
-            *X->aux = *Xs->aux;
+            bmlh_copy_stats(X->aux, Xs->aux);
             single = 0;
         }
     }
@@ -340,7 +340,7 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
             !bmlh_ok(bmlhip_d2d(X->index, Xs->index, (size_t) N * M * sizeof(int)), what) ||
             !bmlh_ok(bmlhip_d2d(X->nnz, Xs->nnz, (size_t) N * sizeof(int)), what))
             goto out;
-        *X->aux = *Xs->aux;
+        bmlh_copy_stats(X->aux, Xs->aux);
     }
     {
         bmlhip_status s;
@@ -359,8 +359,8 @@ void bml_hip_sp2_ellpack(const bml_matrix_ellpack_hip_t *H, bml_matrix_ellpack_h
         *res = r;
 out:
     bmlhip_graph_destroy(graph);
-    bmlhip_free(d_state);
-    bmlhip_free(d_hist);
+    bmlhip_temp_free(d_state);
+    bmlhip_temp_free(d_hist);
     bml_deallocate_ellpack_hip(X2);
     bml_deallocate_ellpack_hip(Xs);
     bml_deallocate_ellpack_hip(X2s);
@@ -382,33 +382,33 @@ static void batch_free(batch_dev *d)
                   d->ab, d->trx, d->trx2, d->norm2, d->norm, d->rowtr, d->rownorm, d->nocc,
                   d->emin, d->emax, d->list, d->qinfo, d->act_off };
     for (size_t k = 0; k < sizeof p / sizeof p[0]; k++)
-        bmlhip_free(p[k]);
+        bmlhip_temp_free(p[k]);
 }
 
 static int batch_alloc(batch_dev *d, int nsys, int N, const char *what)
 {
     memset(d, 0, sizeof *d);
     const size_t S = (size_t) nsys, R = (size_t) N;
-    int ok = bmlh_ok(bmlhip_malloc((void **) &d->row_sys, R * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->row_off, (S + 1) * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->done, S * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->branch, S * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->it, S * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->alldone, 2 * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->stats, 2 * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->ab, 2 * S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->trx, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->trx2, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->norm2, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->norm, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->rowtr, 2 * R * sizeof(double) + 8), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->rownorm, R * sizeof(double) + 8), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->nocc, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->emin, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->emax, S * sizeof(double)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->list, R * sizeof(int) + 8), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->qinfo, 4 * sizeof(int)), what) &&
-             bmlh_ok(bmlhip_malloc((void **) &d->act_off, (S + 1) * sizeof(int)), what);
+    int ok = bmlh_ok(bmlhip_temp_malloc((void **) &d->row_sys, R * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->row_off, (S + 1) * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->done, S * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->branch, S * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->it, S * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->alldone, 2 * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->stats, 2 * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->ab, 2 * S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->trx, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->trx2, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->norm2, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->norm, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->rowtr, 2 * R * sizeof(double) + 8), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->rownorm, R * sizeof(double) + 8), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->nocc, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->emin, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->emax, S * sizeof(double)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->list, R * sizeof(int) + 8), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->qinfo, 4 * sizeof(int)), what) &&
+             bmlh_ok(bmlhip_temp_malloc((void **) &d->act_off, (S + 1) * sizeof(int)), what);
     if (!ok)
         return 0;
     bmlhip_zero(d->done, S * sizeof(int));
@@ -568,8 +568,8 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
 
     /* pack H into one block-diagonal matrix with X's M, then per-system
      * Gershgorin bounds and X0 = (emax I - H)/(emax - emin) */
-    Xc = bml_zero_matrix_ellpack_hip(prec, N, M, X[0]->distribution_mode);
-    X2c = bml_noinit_matrix_ellpack_hip(prec, N, M, X[0]->distribution_mode);
+    Xc = bmlh_temp_matrix_ellpack(prec, N, M, X[0]->distribution_mode);
+    X2c = bmlh_temp_matrix_ellpack(prec, N, M, X[0]->distribution_mode);
     if (!Xc || !X2c)
         goto out;
     {
@@ -605,15 +605,15 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
 
     int single = 0;
     if (o.mixed && o.maxit > o.refine_iters) {
-        Xs = bml_noinit_matrix_ellpack_hip(sprec, N, M, Xc->distribution_mode);
-        X2s = bml_noinit_matrix_ellpack_hip(sprec, N, M, Xc->distribution_mode);
+        Xs = bmlh_temp_matrix_ellpack(sprec, N, M, Xc->distribution_mode);
+        X2s = bmlh_temp_matrix_ellpack(sprec, N, M, Xc->distribution_mode);
         if (!Xs || !X2s)
             goto out;
         if (!bmlh_ok(bmlhip_convert(prec, sprec, (size_t) N * M, Xc->value, Xs->value), what) ||
             !bmlh_ok(bmlhip_d2d(Xs->index, Xc->index, (size_t) N * M * sizeof(int)), what) ||
             !bmlh_ok(bmlhip_d2d(Xs->nnz, Xc->nnz, (size_t) N * sizeof(int)), what))
             goto out;
-        *Xs->aux = *Xc->aux;
+        bmlh_copy_stats(Xs->aux, Xc->aux);
         single = 1;
     }
 
@@ -677,7 +677,7 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
                 !bmlh_ok(bmlhip_d2d(Xc->index, Xs->index, (size_t) N * M * sizeof(int)), what) ||
                 !bmlh_ok(bmlhip_d2d(Xc->nnz, Xs->nnz, (size_t) N * sizeof(int)), what))
                 goto out;
-            *Xc->aux = *Xs->aux;
+            bmlh_copy_stats(Xc->aux, Xs->aux);
             single = 0;
             bmlhip_graph_destroy(graph);
             graph = NULL;
@@ -867,7 +867,7 @@ void bml_hip_sp2_ellblock(const bml_matrix_ellblock_hip_t *H, bml_matrix_ellbloc
                    "of equal block structure and precision", what);
         return;
     }
-    const int prec = X->matrix_precision, NB = X->NB, MB = X->MB;
+    const int prec = X->matrix_precision, MB = X->MB;
     const int sprec = single_of(prec);
     if (o.mixed && !sprec) {
         bmlh_error(BML_HIP_ERR_UNSUPPORTED, "%s: mixed precision needs a double-precision X",
@@ -901,21 +901,19 @@ void bml_hip_sp2_ellblock(const bml_matrix_ellblock_hip_t *H, bml_matrix_ellbloc
     bmlhip_sp2_state *d_state = NULL;
     double *d_hist = NULL;
     /* work matrices: every tile they hold is written before it is read */
-    X2 = bmlh_block_matrix_ellblock_work(prec, NB, MB, X->M, X->bsize_host, X->distribution_mode);
+    X2 = bmlh_temp_matrix_ellblock(X, prec, MB);
     if (!X2)
         goto out;
-    if (!bmlh_ok(bmlhip_malloc((void **) &d_state, sizeof(bmlhip_sp2_state)), what) ||
-        !bmlh_ok(bmlhip_malloc((void **) &d_hist, sizeof(double) * 4 * (size_t) o.maxit), what))
+    if (!bmlh_ok(bmlhip_temp_malloc((void **) &d_state, sizeof(bmlhip_sp2_state)), what) ||
+        !bmlh_ok(bmlhip_temp_malloc((void **) &d_hist, sizeof(double) * 4 * (size_t) o.maxit), what))
         goto out;
     bmlhip_zero(d_state, sizeof(bmlhip_sp2_state));
     bmlhip_zero(d_hist, sizeof(double) * 4 * (size_t) o.maxit);
 
     int single = 0;
     if (o.mixed && o.maxit > o.refine_iters) {
-        Xs = bmlh_block_matrix_ellblock_work(sprec, NB, MB, X->M, X->bsize_host,
-                                             X->distribution_mode);
-        X2s = bmlh_block_matrix_ellblock_work(sprec, NB, MB, X->M, X->bsize_host,
-                                              X->distribution_mode);
+        Xs = bmlh_temp_matrix_ellblock(X, sprec, MB);
+        X2s = bmlh_temp_matrix_ellblock(X, sprec, MB);
         if (!Xs || !X2s || !eb_convert(X, Xs, what))
             goto out;
         single = 1;
@@ -1017,8 +1015,8 @@ void bml_hip_sp2_ellblock(const bml_matrix_ellblock_hip_t *H, bml_matrix_ellbloc
 out:
     if (bmlh_block_engine_setting() != engine0)
         bml_hip_set_block_engine(engine0);
-    bmlhip_free(d_state);
-    bmlhip_free(d_hist);
+    bmlhip_temp_free(d_state);
+    bmlhip_temp_free(d_hist);
     bml_deallocate_ellblock_hip(X2);
     bml_deallocate_ellblock_hip(Xs);
     bml_deallocate_ellblock_hip(X2s);
