@@ -2365,10 +2365,6 @@ struct AddParams {
     const int *row_sys, *sys_done;
     const double *ab_sys;
     int4 *rowstat;  // [N]: (kept, 0, 0, 0), kept = -1 for a skipped row
-    // batched work queue (NULL: one block per row): rows qlist[0 ..
-    // qinfo[0]), taken with the cursor qinfo[2]
-    const int *qlist;
-    int *qinfo;
 };
 
 // tsize: any table size; a column's home slot is its multiplicative hash
@@ -2461,42 +2457,151 @@ __device__ void add_row(const AddParams &p, int i, int *keys, T *xs, T *ys, ORD 
     }
 }
 
+// A <- alpha A + beta B, a wavefront per row.  Only A's columns are hashed
+// (column -> position in A's row, 6 bytes a slot); B's entries look
+// themselves up and leave their own position with A's entry, or go on the
+// list of new columns.  The values stay in global memory and are read once,
+// in the passes that write the row: A's entries in A's order, then the new
+// ones in B's order, which is the union order of the reference
+// (bml_add_ellpack_typed.c:162-196).
+//
+// Memory bound: the rows of A and B once in, A's once out.  The former
+// kernel kept keys, both value sums and the order of the whole union in LDS
+// (24 KB a row at M = 264, six wavefronts per CU; this one needs 4 KB):
+// 32^3 lattice step (177 entries a row, double) 165 -> 59 us,
+// a batch of 38394 rows 474 -> 50 us.
+//
+// The row's norm sums run over the union in 64 strides as before, so it
+// rounds the same.  Entries are overwritten at or before the position they
+// were read from, a chunk's reads before its writes.
+constexpr int ADD_WAVES = 4;
+constexpr size_t add_row_bytes(int tbits, int MA, int MB) {
+    return ((size_t) 6 << tbits) + (((size_t) 2 * (MA + MB) + 15) & ~(size_t) 15);
+}
+
 template <typename T>
-__global__ __launch_bounds__(64) void k_add_lds(AddParams p, unsigned tsize) {
+__global__ __launch_bounds__(64 * ADD_WAVES) void k_add_rows(AddParams p, int tbits) {
+    using E = Elem<T>;
     extern __shared__ __align__(16) unsigned char smem[];
     if (p.skip && *p.skip) return;
-    T *xs = (T *) smem;
-    T *ys = xs + tsize;
-    int *keys = (int *) (ys + tsize);
-    uint16_t *ord = (uint16_t *) (keys + tsize);
-    for (unsigned s = threadIdx.x; s < tsize; s += 64) {
-        keys[s] = EMPTY;
-        xs[s] = Elem<T>::zero();
-        ys[s] = Elem<T>::zero();
-    }
-    __syncthreads();
-    if (p.qlist) {
-        // persistent over the work queue (each row leaves the table clean;
-        // the next take is issued while the current row runs)
-        const int n = p.qinfo[0];
-        int q = 0;
-        if (threadIdx.x == 0) q = atomicAdd(&p.qinfo[2], 1);
-        q = __shfl(q, 0, 64);
-        while (q < n) {
-            int nxt = 0;
-            if (threadIdx.x == 0) nxt = atomicAdd(&p.qinfo[2], 1);
-            add_row<T, uint16_t>(p, p.qlist[q], keys, xs, ys, ord, tsize);
-            __syncthreads();
-            q = __shfl(nxt, 0, 64);
-        }
-        return;
-    }
-    const int i = blockIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6), lane = lane_id();
+    const int i = blockIdx.x * (blockDim.x >> 6) + w;
+    if (i >= p.N) return;
     if (p.row_sys && p.sys_done[p.row_sys[i]]) {
-        if (threadIdx.x == 0) p.rowstat[i] = make_int4(-1, 0, 0, 0);
+        if (lane == 0) p.rowstat[i] = make_int4(-1, 0, 0, 0);
         return;
     }
-    add_row<T, uint16_t>(p, i, keys, xs, ys, ord, tsize);
+    const unsigned ts = 1u << tbits;
+    int *keys = (int *) (smem + w * add_row_bytes(tbits, p.MA, p.MB));
+    uint16_t *pos = (uint16_t *) (keys + ts);
+    uint16_t *from = pos + ts;         // [MA] B's entry at A's column (NONE: none)
+    uint16_t *fresh = from + p.MA;     // [MB] B's entries at columns that A lacks
+    constexpr unsigned NONE = 0xFFFFu;
+    const uint64_t ltmask = (1ull << lane) - 1ull;
+    T *Av = (T *) p.Av;
+    const T *Bv = (const T *) p.Bv;
+    const size_t rA = (size_t) i * p.MA, rB = (size_t) i * p.MB;
+    const double *ab = p.ab_sys ? p.ab_sys + 2 * p.row_sys[i] : p.ab;
+    const double alpha = ab ? ab[0] : p.alpha;
+    const double beta = ab ? ab[1] : p.beta;
+    // without a norm, a matrix times zero adds no columns
+    const bool usea = p.mode != 0 || alpha > 0.0 || alpha < 0.0;
+    const bool useb = p.mode != 0 || beta > 0.0 || beta < 0.0;
+    const int nA = usea ? p.An[i] : 0, nB = useb ? p.Bn[i] : 0;
+    for (unsigned s = lane; s < ts / 4; s += 64)
+        reinterpret_cast<int4 *>(keys)[s] = make_int4(EMPTY, EMPTY, EMPTY, EMPTY);
+    __builtin_amdgcn_wave_barrier();
+    for (int k0 = 0; k0 < nA; k0 += 64) {
+        const int kp = k0 + lane;
+        if (kp < nA) {
+            const int col = p.Ai[rA + kp];
+            from[kp] = (uint16_t) NONE;
+            unsigned h = hash_slot(col, tbits);
+            while (atomicCAS(&keys[h], EMPTY, col) != EMPTY) h = (h + 1u) & (ts - 1u);
+            pos[h] = (uint16_t) kp;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    int nnew = 0;
+    for (int k0 = 0; k0 < nB; k0 += 64) {
+        const int kp = k0 + lane;
+        bool isnew = false;
+        if (kp < nB) {
+            const int col = p.Bi[rB + kp];
+            unsigned h = hash_slot(col, tbits);
+            int k;
+            while ((k = keys[h]) != col && k != EMPTY) h = (h + 1u) & (ts - 1u);
+            isnew = k != col;
+            if (!isnew) from[pos[h]] = (uint16_t) kp;
+        }
+        const uint64_t nm = __builtin_amdgcn_ballot_w64(isnew);
+        if (isnew) fresh[nnew + popc64(nm & ltmask)] = (uint16_t) kp;
+        nnew += popc64(nm);
+    }
+    __builtin_amdgcn_wave_barrier();
+    int kept = 0;
+    double nrm = 0.0;
+    auto emit = [&](bool act, int col, T x, T y) __attribute__((always_inline)) {
+        if (p.mode == 1 && act) nrm += E::re_sq(y);
+        if (p.mode == 2 && act) nrm += E::abs2(y);
+        const uint64_t km = __builtin_amdgcn_ballot_w64(act && E::above(x, p.thr));
+        const int at = kept + popc64(km & ltmask);
+        if (act && E::above(x, p.thr) && at < p.MA) {
+            p.Ai[rA + at] = col;
+            Av[rA + at] = x;
+        }
+        kept += popc64(km);
+    };
+    // (the next chunk of A's row is read before this one is written)
+    int col = 0, ncol = 0;
+    T av = E::zero(), nav = E::zero();
+    if (lane < nA) {
+        col = p.Ai[rA + lane];
+        av = Av[rA + lane];
+    }
+    for (int k0 = 0; k0 < nA; k0 += 64) {
+        const int kp = k0 + lane;
+        const bool act = kp < nA;
+        if (kp + 64 < nA) {
+            ncol = p.Ai[rA + kp + 64];
+            nav = Av[rA + kp + 64];
+        }
+        T x = E::zero(), y = E::zero();
+        if (act) {
+            const unsigned f = from[kp];
+            const T bv = f != NONE ? Bv[rB + f] : E::zero();
+            x = E::axpy(x, alpha, av);
+            if (p.mode) y = E::add(y, av);
+            if (f != NONE) {
+                x = E::axpy(x, beta, bv);
+                if (p.mode) y = E::sub(y, bv);
+            }
+        }
+        emit(act, col, x, y);
+        col = ncol;
+        av = nav;
+    }
+    for (int r0 = nA & ~63; r0 < nA + nnew; r0 += 64) {
+        const int r = r0 + lane;
+        const bool act = r >= nA && r < nA + nnew;
+        T x = E::zero(), y = E::zero();
+        int c = 0;
+        if (act) {
+            const int kp = fresh[r - nA];
+            c = p.Bi[rB + kp];
+            const T bv = Bv[rB + kp];
+            x = E::axpy(x, beta, bv);
+            if (p.mode) y = E::sub(y, bv);
+        }
+        emit(act, c, x, y);
+    }
+    // fixed-order wavefront reduction of the row's norm
+    for (int off = 32; off > 0; off >>= 1) nrm += __shfl_down(nrm, off, 64);
+    if (lane == 0) {
+        p.An[i] = kept < p.MA ? kept : p.MA;
+        p.rowstat[i] = make_int4(kept, 0, 0, 0);
+        if (p.mode) p.rownorm[i] = nrm;
+    }
 }
 
 template <typename T>
@@ -3430,26 +3535,25 @@ int add_typed(int N, int MA, void *Av, int *Ai, int *An, int MB, const void *Bv,
     p.row_sys = batch ? batch->d_row_sys : nullptr;
     p.sys_done = batch ? batch->d_done : nullptr;
     p.ab_sys = batch ? batch->d_ab : nullptr;
-    p.qlist = batch ? batch->d_list : nullptr;
-    p.qinfo = batch ? batch->d_qinfo : nullptr;
     p.st = bmlhip_status_dev();
     p.rownorm = rownorm ? rownorm : (double *) bmlhip_scratch(0, sizeof(double) * (size_t) (N + 1));
     p.rowstat = (int4 *) bmlhip_scratch(BMLHIP_ROWSTAT_SLOT, sizeof(int4) * (size_t) (N + 1));
     if (!p.rownorm || !p.rowstat) return 4;
     int rc = bmlhip_status_ready();
     if (rc) return rc;
-    // a row's union has at most MA + MB columns: the LDS table keeps it at
-    // most 4/5 full (multiple of 64 slots; first-touch list in 16 bits)
+    // the table holds A's columns at most two thirds full; positions are 16
+    // bits
+    const int abits = ceil_log2((long long) MA * 3 / 2 + 32);
+    const size_t row = add_row_bytes(abits, MA, MB);
+    // (the global-table pass: a row's union has at most MA + MB columns)
     const int tbits = ceil_log2((long long) (MA + MB) * 4 / 3 + 64);
     const size_t lds = ((size_t) 1 << tbits) * (2 * sizeof(T) + 2 * sizeof(int));
-    const unsigned tl = (unsigned) (((long long) (MA + MB) * 5 / 4 + 64 + 63) & ~63ll);
-    const size_t lds_l = (size_t) tl * (2 * sizeof(T) + sizeof(int) + sizeof(uint16_t));
     if (N > 0) {
-        if (lds_l <= 64 * 1024 && tl < 65536) {
-            const int blocks = !p.qlist ? N
-                               : persistent_blocks((const void *) k_add_lds<T>, 64, lds_l, N);
-            hipLaunchKernelGGL(k_add_lds<T>, dim3(blocks), dim3(64), lds_l, s, p, tl);
-            if ((rc = report("k_add_lds"))) return rc;
+        if (row <= 64 * 1024 && MA < 65535 && MB < 65535) {
+            const int waves = row * ADD_WAVES <= 32 * 1024 ? ADD_WAVES : 1;
+            hipLaunchKernelGGL(k_add_rows<T>, dim3((N + waves - 1) / waves), dim3(64 * waves),
+                               row * waves, s, p, abits);
+            if ((rc = report("k_add_rows"))) return rc;
         } else {
             const int blocks = 256;
             unsigned char *tabs = (unsigned char *) bmlhip_scratch(2, blocks * lds + 256);
