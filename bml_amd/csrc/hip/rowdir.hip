@@ -1,8 +1,9 @@
 // Row products on directly indexed accumulators: the exact engine's kernel
 // for all but very wide matrices.
 //
-// A block of W wavefronts forms RB = W * 64/GROUP consecutive output rows, a
-// group of GROUP lanes per row.  The columns the block's rows can touch are
+// W wavefronts of a block form RB = W * 64/GROUP consecutive output rows, a
+// group of GROUP lanes per row (wavefronts beyond W help with steps 1 to 3
+// below and end: where few rows fit a CU, its SIMDs would idle meanwhile).  The columns the block's rows can touch are
 // found first and numbered in column order; a row's running sums then lie in
 // an LDS array with one slot per such column, and a product's slot is
 //
@@ -29,7 +30,8 @@
 //
 // Measured on one MI355X against the hash-table kernels (double unless said):
 // 32^3 lattice iterate squared (177 entries a row, 1.03e9 products) 4.71 ->
-// 1.94 ms; 24^3 complex double (279 a row, 1.08e9 products) 10.5 -> 6.7 ms;
+// 1.81 ms (1.94 without helpers); 24^3 complex double (279 a row, 1.08e9
+// products) 10.5 -> 5.5 ms (6.7);
 // random banded N = 4096 (31 a row) 112 -> 37 us; N = 500 137 -> 12.6 us;
 // single precision A B of N = 10007 with C merged 181 -> 70 us.
 //
@@ -187,14 +189,14 @@ constexpr int pipe_depth() { return NCH == 1 ? 8 : (NCH <= 3 ? 6 : 4); }
 
 template <typename T, int GROUP, int NCH>
 __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_bytes, int nwcap,
-                                                    int mode) {
+                                                    int mode, int W) {
     using E = Elem<T>;
     constexpr int RW = 64 / GROUP;  // rows per wavefront
     constexpr int PD = pipe_depth<NCH>();
     constexpr int S = NCH * GROUP;  // entries of a row of B per step
     extern __shared__ __align__(16) unsigned char smem[];
     if (p.skip && *p.skip) return;
-    const int tid = threadIdx.x, T_ = blockDim.x, W = T_ >> 6;
+    const int tid = threadIdx.x, T_ = blockDim.x, H = T_ >> 6;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane / GROUP, gl = lane % GROUP;
     const uint64_t gmask = GROUP == 64 ? ~0ull : (((1ull << GROUP) - 1ull) << (g * GROUP));
     const uint64_t ltmask = (1ull << lane) - 1ull;
@@ -291,7 +293,9 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
             cb = some;
         }
     };
-    begin_row(row_of(w * RW + g));
+    // (helpers of a single row know it too)
+    const bool own = mode == BMLHIP_DIR_OWN, shared_row = own && W == 1;
+    begin_row(w < W || shared_row ? row_of((shared_row ? 0 : w) * RW + g) : -1);
 
     // columns the rows can reach: all, or those of the systems of the
     // block's first and last row (the systems between them too)
@@ -332,10 +336,9 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
             const unsigned bit = 1u << (kk & 31);
             if (act && !(*word & bit)) atomicOr(word, bit);
         };
-        auto mark_rows = [&](unsigned rb, int n, int count, bool own)
-                             __attribute__((always_inline)) {
-            const int stride = own ? Q : Q * RW;
-            for (int t = 0; t < count; t += stride) {
+        auto mark_rows = [&](unsigned rb, int n, int count) __attribute__((always_inline)) {
+            const int stride = own ? (shared_row ? H * Q : Q) : Q * RW;
+            for (int t = shared_row ? w * Q : 0; t < count; t += stride) {
                 int kcol[Q][NCH], nq[Q];
                 unsigned rq[Q];
 #pragma unroll
@@ -364,7 +367,6 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
                 }
             }
         };
-        const bool own = mode == BMLHIP_DIR_OWN;
         unsigned *jbits = (unsigned *) pool;
         for (int k = tid; k < nw; k += T_) {
             idx[k] = make_uint2(0u, 0u);
@@ -373,12 +375,12 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
         if (tid == 0) list_s = 0;
         __syncthreads();
         if (own) {
-            mark_rows(cb, cn, steps < GROUP ? steps : GROUP, true);
+            mark_rows(cb, cn, steps < GROUP ? steps : GROUP);
             for (int t0 = GROUP; t0 < steps; t0 += GROUP) {
                 const int e = t0 + gl;
                 const int j = e < nA ? Ai[rowA + (unsigned) e] : -1;
                 mark_rows((unsigned) (j >= 0 ? j : 0) * MB, j >= 0 ? Bn[j] : 0,
-                          steps - t0 < GROUP ? steps - t0 : GROUP, true);
+                          steps - t0 < GROUP ? steps - t0 : GROUP);
             }
         } else {
             int *jlist = (int *) (pool + up16(4u * (unsigned) nw));
@@ -404,12 +406,12 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
             const int U = list_s;
             fits = U <= jcap;
             if (fits) {
-                const int share = (U + W - 1) / W;
+                const int share = (U + H - 1) / H;
                 const int u1 = (w + 1) * share < U ? (w + 1) * share : U;
                 for (int u0 = w * share; u0 < u1; u0 += 64) {
                     const int n = u1 - u0 < 64 ? u1 - u0 : 64;
                     const int jl = lane < n ? jlist[u0 + lane] : jlist[u0];
-                    mark_rows((unsigned) jl * MB, lane < n ? Bn[jl] : 0, n, false);
+                    mark_rows((unsigned) jl * MB, lane < n ? Bn[jl] : 0, n);
                 }
             }
         }
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
             if (lane == 63) part_s[w] = inc;
             __syncthreads();
             int at = inc - n;
-            for (int v = 0; v < W; v++) {
+            for (int v = 0; v < H; v++) {
                 const int pv = __builtin_amdgcn_readfirstlane(part_s[v]);
                 if (v < w) at += pv;
                 D += pv;
@@ -445,7 +447,7 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
     // 2^16 columns or more, its slot, with colof[slot] beside it.
     const bool wide = span > 65536;
     const unsigned fixed =
-        (wide ? up16(4u * (unsigned) D) : 0u) + (unsigned) T_ * (unsigned) sizeof(T);
+        (wide ? up16(4u * (unsigned) D) : 0u) + 64u * (unsigned) W * (unsigned) sizeof(T);
     const unsigned per_row = up16((unsigned) (D * (int) sizeof(T))) + up16(2u * (unsigned) D);
     int nconc = 0;
     if (fits && D <= 65535 && fixed < pool_bytes)
@@ -453,6 +455,7 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
     if (nconc > RB) nconc = RB;
     if (nconc == 0) {
         const int r = w * RW + g;
+        if (w >= W) return;
         if (gl == 0 && i >= 0) {
             const int q = atomicAdd(&p.st->table_overflow_rows, 1);
             p.ovf[q] = i;
@@ -482,6 +485,7 @@ __global__ __launch_bounds__(512) void k_spgemm_dir(SpParams p, unsigned lds_byt
       }
       __syncthreads();
     }
+    if (w >= W) return;
     *priv = E::zero();
 
     const bool haveslots = w * RW + g < nconc;
@@ -666,17 +670,33 @@ int fail(const char *what, hipError_t e) {
     return 3;
 }
 
+// wavefronts of a kernel that a CU's registers hold, at most 16
+int resident(const void *fn) {
+    hipFuncAttributes at;
+    if (hipFuncGetAttributes(&at, fn) != hipSuccess || at.numRegs <= 0) return 8;
+    const int n = 4 * (512 / ((at.numRegs + 7) / 8 * 8));
+    return n < 4 ? 4 : (n > 16 ? 16 : n);
+}
+
 template <typename T, int GROUP, int NCH>
 int launch(const SpParams &p, int waves, int lds, int span, int mode, hipStream_t s) {
     const int RB = waves * (64 / GROUP);
     const void *fn = (const void *) k_spgemm_dir<T, GROUP, NCH>;
+    // helpers up to what a CU holds, where the columns are found and all
+    // wavefronts can take part
+    int all = waves;
+    if (mode == BMLHIP_DIR_LIST || (mode == BMLHIP_DIR_OWN && RB == 1)) {
+        static const int most = resident(fn);
+        const int blocks = 160 * 1024 / lds;
+        while (all < 8 && (all + 1) * blocks <= most) all++;
+    }
     if (lds > 64 * 1024)
         (void) hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     const int nblk = (p.N + RB - 1) / RB;
     if (nblk > 0) {
         bmlhip_prof_mark_begin(PrecOf<T>::value);
-        hipLaunchKernelGGL((k_spgemm_dir<T, GROUP, NCH>), dim3(nblk), dim3(64 * waves), lds, s,
-                           p, (unsigned) lds, span / 32 + 2, mode);
+        hipLaunchKernelGGL((k_spgemm_dir<T, GROUP, NCH>), dim3(nblk), dim3(64 * all), lds, s,
+                           p, (unsigned) lds, span / 32 + 2, mode, waves);
         bmlhip_prof_mark_end();
     }
     const hipError_t e = hipGetLastError();
