@@ -58,6 +58,9 @@ constexpr int NUM_WAVES = BMLHIP_EB_WAVES;  // wavefronts per block row in k_eb_
 // for the symmetric X^2 of the 16x16x8-site, 32-orbital lattice; 2 or 8
 // wavefronts per block row ran 10-20% slower than 4.
 constexpr int EB_BATCH = BMLHIP_EB_BATCH;
+constexpr int STREAM_BATCH = 8;  // and for k_eb_stream (see there)
+constexpr int EB_QUEUES = 8;  // k_eb_stream: one queue of batches per XCD,
+constexpr int EB_HEAD = 64;   // their heads this many ints apart
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef double doublex4 __attribute__((ext_vector_type(4)));
@@ -82,20 +85,22 @@ struct EbParams {
     int *soff;       // [NB*(maxs+1)] start of each slot's pair list
     int *pairs;      // [NB*maxp] jp << 16 | kp, grouped by slot
     int *pslot;      // [NB*maxp] slot of each pair
-    int *bfirst;     // [NB*(maxp/EB_BATCH+2)] batch k: slots [bfirst[k], bfirst[k+1])
+    int batch;       // pairs per batch: EB_BATCH or STREAM_BATCH
+    int *bfirst;     // [NB*(maxp/batch+2)] batch k: pairs [bfirst[k], bfirst[k+1])
+    int *nbat;       // [NB] batches of each block row, then the 8 queue heads of k_eb_stream
+    int head0;       // where the heads start: the wavefronts that begin at each queue
     double *rowtr;   // [2*NB] per block row tr X, tr X^2 (x2)
     int4 *rowstat;   // [NB] (kept, touched, block pairs, nnzb of A's row)
     bmlhip_status *st;
     const int *skip;
     int remap;  // numeric pass: XCD-aware block-row order (xcd_block)
     int sym;    // x2 of an exactly symmetric X: each row forms the slots it owns (sym_owner)
-    int *kflag; // [NB*maxs] sym: kept flag of every slot, set by its row or its mirror
+    int *kflag; // [NB*maxs] sym, k_eb_stream: kept flag of every slot, set by its row or its mirror
     const __bf16 *A16, *B16;  // bf16 engine: A's tiles row-major, B's transposed (k_eb_bf16)
     int ka;  // MFMA engines: the first ka A tiles of a block row are staged in LDS
     // fused SP2 update (sym x2 on an MFMA engine): C <- ab[0] X + ab[1] X^2,
-    // A's block columns in LDS at byte acol_off of the dynamic area, the
-    // rows' |X - X^2|^2 into rownorm
-    int fuse, acol_off;
+    // |X - X^2|^2 and the next traces of each workgroup into rownorm
+    int fuse;
     const double *ab;
     double *rownorm;
 };
@@ -247,18 +252,25 @@ __global__ __launch_bounds__(64) void k_eb_symbolic(EbParams p, int tbits, int c
     if (lane == 0) off[count] = running;
     // the loop below reads fill[s - 1], written by lane s - 1 above
     __syncthreads();
-    // batch starts: bfirst[k] = the first slot s with off[s] >= EB_BATCH k
-    // (count for the end), k <= running / EB_BATCH + 1
-    int *bf = p.bfirst + (size_t) ib * (p.maxp / EB_BATCH + 2);
+    // batch starts: bfirst[k] = off[s] of the first slot s with
+    // off[s] >= batch k (the row's pair count for the end),
+    // k <= running / batch + 1
+    int *bf = p.bfirst + (size_t) ib * (p.maxp / p.batch + 2);
     for (int s0 = 0; s0 <= count; s0 += 64) {
         const int s = s0 + lane;
         if (s <= count) {
             const int cur = s < count ? fill[s] : running;
-            const int klo = s == 0 ? 0 : fill[s - 1] / EB_BATCH + 1;
-            for (int k = klo; k <= cur / EB_BATCH; k++) bf[k] = s;
+            const int klo = s == 0 ? 0 : fill[s - 1] / p.batch + 1;
+            for (int k = klo; k <= cur / p.batch; k++) bf[k] = cur;
         }
     }
-    if (lane == 0) bf[running / EB_BATCH + 1] = count;
+    if (lane == 0) {
+        bf[running / p.batch + 1] = running;
+        p.nbat[ib] = running > 0 ? running / p.batch + 1 : 0;
+        if (ib == 0)
+            for (int x = 0; x < EB_QUEUES; x++) p.nbat[p.NB + x * EB_HEAD] = p.head0;
+        if (p.kflag && !p.fuse && p.kind == 0) p.rowtr[ib] = p.rowtr[p.NB + ib] = 0.0;
+    }
     __syncthreads();
     // pass 2: pairs grouped by slot, jp order kept within a slot
     int *pr = p.pairs + (size_t) ib * p.maxp;
@@ -283,7 +295,7 @@ __global__ __launch_bounds__(64) void k_eb_symbolic(EbParams p, int tbits, int c
             __syncthreads();
         }
     }
-    if (p.sym)
+    if (p.kflag)
         for (int q = lane; q < count; q += 64) p.kflag[(size_t) ib * p.maxs + q] = 0;
     // the numeric pass records the row's counts (touched > MC is an overflow)
     if (lane == 0) p.cnt[ib] = count;
@@ -355,6 +367,7 @@ template <typename X> __device__ __forceinline__ X gld(const X *a) {
     return *(const __attribute__((address_space(1))) X *) a;
 }
 template <typename X> using lds_ptr = const __attribute__((address_space(3))) X *;
+using lds_tile = __attribute__((address_space(3))) double *;
 
 // MFMA engine, single real, 32 x 32 tiles: v_mfma_f32_32x32x2f32 takes a
 // 32x2 slice of L (lane l: row l%32) and a 2x32 slice of R (lane l: column
@@ -528,13 +541,18 @@ __global__ __launch_bounds__(256) void k_eb_bf16(int M, const float *V, const in
 // MFMA engine, double real, 32 x 32 tiles as 2 x 2 tiles of 16 x 16:
 // v_mfma_f64_16x16x4f64 takes a 16x4 slice of L (lane l: row l%16, k group
 // l/16) and a 4x16 slice of R.  Step s pairs k = 8g + s for the four lane
-// groups g, so a lane reads 8 contiguous elements of its row of L.  Output:
-// lane l, register v holds row l/16 + 4v, column l%16 of its 16x16 tile.
+// groups g; of the two tiles side by side, tile tj holds columns 2c + tj, so
+// a lane's elements of a row of R are one 16-byte load.  Output: lane l,
+// register v holds row l/16 + 4v, column 2(l%16) + tj.
+//
+// The matrix unit wants the left tile by rows, 16 of them per instruction,
+// 256 bytes apart.  It is loaded as it lies (whole lines) and turned in LDS
+// (put, then mma): row r keeps its 16-byte chunk c at c ^ (r & 15), so the 16
+// lanes that read one chunk of 16 rows hit 16 different bank groups.
 struct MfmaAccF64 {
-    static constexpr bool kPipelined = true;
     doublex4 a[2][2];
     struct Frag {
-        double lv[2][8], rv[2][8];
+        doublex2 l[8], r[8];
     };
     __device__ void zero() {
 #pragma unroll
@@ -548,60 +566,37 @@ struct MfmaAccF64 {
         const int lane = lane_id();
         const int c = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int ti = 0; ti < 2; ti++) {
-            const doublex2 *l2 = reinterpret_cast<const doublex2 *>(L + (ti * 16 + c) * 32 + g * 8);
+        for (int q = 0; q < 8; q++) f.l[q] = gld(reinterpret_cast<const doublex2 *>(L) + 64 * q + lane);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const doublex2 t = gld(l2 + q);
-                f.lv[ti][2 * q] = t[0];
-                f.lv[ti][2 * q + 1] = t[1];
-            }
-        }
-#pragma unroll
-        for (int tj = 0; tj < 2; tj++)
-#pragma unroll
-            for (int s = 0; s < 8; s++) f.rv[tj][s] = gld(R + (g * 8 + s) * 32 + tj * 16 + c);
+        for (int s = 0; s < 8; s++) f.r[s] = gld(reinterpret_cast<const doublex2 *>(R + (g * 8 + s) * 32) + c);
     }
-    // A tile staged in LDS: row r (256 bytes, 16 chunks) keeps chunk c at
-    // c ^ (r & 7)
-    using TA = double;
-    // not staged: two blocks per CU leave room for 5 FP64 tiles, and the
-    // second load path costs the pipelined loop its last registers
-    static constexpr bool kStage = false;
-    static constexpr int kChunks = 16;
-    __device__ static int swz(int r, int c) { return c ^ (r & 7); }
-    __device__ static void load_s(lds_ptr<double> Ls, const double *R, Frag &f) {
+    __device__ static void put(lds_tile t, const Frag &f) {
         const int lane = lane_id();
         const int c = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int ti = 0; ti < 2; ti++) {
-            const int r = ti * 16 + c;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const doublex2 t = *(lds_ptr<doublex2>) (Ls + r * 32 + 2 * swz(r, 4 * g + q));
-                f.lv[ti][2 * q] = t[0];
-                f.lv[ti][2 * q + 1] = t[1];
-            }
+        for (int q = 0; q < 8; q++) {
+            const int r = 4 * q + g;
+            *(__attribute__((address_space(3))) doublex2 *) (t + r * 32 + 2 * (c ^ (r & 15))) = f.l[q];
         }
-#pragma unroll
-        for (int tj = 0; tj < 2; tj++)
-#pragma unroll
-            for (int s = 0; s < 8; s++) f.rv[tj][s] = gld(R + (g * 8 + s) * 32 + tj * 16 + c);
     }
-    __device__ void mma(const Frag &f) {
+    __device__ void mma(lds_tile t, const doublex2 (&rt)[8]) {
+        const int lane = lane_id();
+        const int c = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int s = 0; s < 8; s++)
+        for (int q = 0; q < 4; q++) {
+            doublex2 lv[2];
 #pragma unroll
             for (int ti = 0; ti < 2; ti++)
+                lv[ti] = *(lds_ptr<doublex2>) (t + (ti * 16 + c) * 32 + 2 * ((4 * g + q) ^ c));
 #pragma unroll
-                for (int tj = 0; tj < 2; tj++)
-                    a[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.lv[ti][s], f.rv[tj][s],
-                                                                     a[ti][tj], 0, 0, 0);
-    }
-    __device__ void mac(const double *L, const double *R, int, int, int) {
-        Frag f;
-        load(L, R, f);
-        mma(f);
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int ti = 0; ti < 2; ti++)
+#pragma unroll
+                    for (int tj = 0; tj < 2; tj++)
+                        a[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(lv[ti][e], rt[2 * q + e][tj],
+                                                                         a[ti][tj], 0, 0, 0);
+        }
     }
     __device__ double maxmag() const {
         double m = 0.0;
@@ -619,25 +614,32 @@ struct MfmaAccF64 {
 #pragma unroll
         for (int ti = 0; ti < 2; ti++)
 #pragma unroll
-            for (int tj = 0; tj < 2; tj++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) C[(ti * 16 + g + 4 * v) * ld + tj * 16 + c] = a[ti][tj][v];
+            for (int v = 0; v < 4; v++) {
+                double *row = C + (ti * 16 + g + 4 * v) * ld + 2 * c;
+                if (ld % 2 == 0) {  // rows of whole 16-byte chunks
+                    *reinterpret_cast<doublex2 *>(row) = doublex2{a[ti][0][v], a[ti][1][v]};
+                } else {
+                    row[0] = a[ti][0][v];
+                    row[1] = a[ti][1][v];
+                }
+            }
     }
     __device__ void diag(double *dg) const {
         const int lane = lane_id();
         const int c = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int ti = 0; ti < 2; ti++)
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                if (g + 4 * v == c) dg[t * 16 + c] = a[t][t][v];
+            for (int tj = 0; tj < 2; tj++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (ti * 16 + g + 4 * v == 2 * c + tj) dg[2 * c + tj] = a[ti][tj][v];
     }
 };
 
 template <typename T, int ENGINE, int BT> struct AccOf { using type = ExactAcc<T, BT>; };
 template <> struct AccOf<float, 1, 32> { using type = MfmaAccF32; };
 template <> struct AccOf<float, 2, 32> { using type = MfmaAccBF16; };
-template <> struct AccOf<double, 1, 32> { using type = MfmaAccF64; };
 
 // lane src's value (src wave-uniform): two scalar reads of the halves
 __device__ __forceinline__ size_t lane_get(size_t v, int src) {
@@ -761,6 +763,110 @@ __device__ __forceinline__ int mirror_slot(const EbParams &p, const MirrorProbe 
     return -1;
 }
 
+// The end of a finished tile of a symmetric X^2 (slot s of row ib, block
+// column kb, its max |element| already tested: keep): the fused update where
+// asked for, the kept flag of the slot and of its mirror, the tile at (ib, s)
+// and its transpose at (kb, s').  stg is this wavefront's staging tile;
+// xl(jx, e) gives element e of X's block jx of row ib.
+template <typename T, int BT, typename Acc, typename XL>
+__device__ __forceinline__ void finish_sym(const EbParams &p, const Acc &acc, int ib, int s, int kb,
+                                           const MirrorProbe &mp, T *stg, bool keep, int nAr, double alpha,
+                                           double beta, double &nrm_l, double &frob_l, double &trn_l, XL xl) {
+    using E = Elem<T>;
+    constexpr size_t B2 = (size_t) BT * BT;
+    constexpr int LD = BT + 1;
+    const int lane = threadIdx.x % 64;
+    T *Cv = (T *) p.Cv;
+    const int sp = kb != ib ? mirror_slot(p, mp, kb, ib) : -1;
+    auto wave_sync = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    bool kept = keep;
+    if (p.fuse) {
+        // U = alpha X[ib, kb] + beta Y, Y the product's block when the x2
+        // rule keeps it (else 0), formed in the staging tile; U kept iff
+        // it is the diagonal block or max |U| > thr (the add's rule;
+        // every X block is reached through its row's diagonal block, so
+        // none is left out); |X - Y|^2 counted twice off the diagonal
+        // (the mirror block)
+        acc.store(stg, LD);
+        wave_sync();
+        if (kb == ib) {  // the diagonal block takes its upper triangle
+            for (int e = lane; e < (int) B2; e += 64) {
+                const int r = e / BT, c = e % BT;
+                if (r > c) stg[r * LD + c] = E::conj(stg[c * LD + r]);
+            }
+            wave_sync();
+        }
+        // the row's own block columns hold the first slots, in A's order
+        const int jx = s < nAr ? s : -1;
+        constexpr int QE = (int) (B2 / 64);
+        static_assert(B2 % 64 == 0, "a tile is whole rows of 64 lanes");
+        // chunks of a lane's elements, each chunk's loads issued before any
+        // is used: all of them for 4-byte elements, two at a time for 8-byte
+        // ones, whose kernel has no registers to spare (16 spilled, and were
+        // no faster)
+        constexpr int CH = sizeof(T) <= 4 ? QE : (QE >= 2 ? 2 : QE);
+        double mu = 0.0, dn = 0.0, fu = 0.0, tu = 0.0;
+#pragma unroll 1
+        for (int q0 = 0; q0 < QE; q0 += CH) {
+            T xv[CH];
+#pragma unroll
+            for (int j = 0; j < CH; j++) xv[j] = jx >= 0 ? xl(jx, lane + 64 * (q0 + j)) : E::zero();
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                const int e = lane + 64 * (q0 + j), r = e / BT, c = e % BT;
+                const T y = keep ? stg[r * LD + c] : E::zero();
+                const T u = E::axpy(E::axpy(E::zero(), alpha, xv[j]), beta, y);
+                stg[r * LD + c] = u;
+                mu = fmax(mu, E::mag(u));
+                dn += E::abs2(E::sub(xv[j], y));
+                fu += E::abs2(u);
+                if (r == c) tu += E::re(u);
+            }
+        }
+        nrm_l += kb == ib ? dn : 2.0 * dn;
+        kept = kb == ib || wave_max(mu) > p.thr;
+        if (kept && (s < p.MC || (sp >= 0 && sp < p.MC))) {
+            frob_l += kb == ib ? fu : 2.0 * fu;
+            if (kb == ib) trn_l += tu;
+        }
+        wave_sync();
+    }
+    if (lane == 0) {
+        p.kflag[(size_t) ib * p.maxs + s] = kept;
+        if (sp >= 0) p.kflag[(size_t) kb * p.maxs + sp] = kept;
+    }
+    if (kept && (s < p.MC || (sp >= 0 && sp < p.MC))) {
+        if (!p.fuse) {
+            acc.store(stg, LD);
+            wave_sync();
+        }
+        if (s < p.MC) {
+            const size_t sc = (size_t) ib * p.MC + s;
+            T *D = Cv + sc * B2;
+            for (int e = lane; e < (int) B2; e += 64) {
+                const int r = e / BT, c = e % BT;
+                D[e] = (kb == ib && r > c) ? E::conj(stg[c * LD + r]) : stg[r * LD + c];
+            }
+            if (lane == 0) p.Ci[sc] = kb;
+        }
+        if (sp >= 0 && sp < p.MC) {
+            const size_t sc = (size_t) kb * p.MC + sp;
+            T *D = Cv + sc * B2;
+            for (int e = lane; e < (int) B2; e += 64) {
+                const int r = e / BT, c = e % BT;
+                D[e] = E::conj(stg[c * LD + r]);
+            }
+            if (lane == 0) p.Ci[sc] = ib;
+        }
+        // the staging tile is read before the next slot overwrites it
+        wave_sync();
+    }
+}
+
 // blocks per CU the registers are held to: 3 for the bf16 engine (its
 // 48 KB LDS share leaves room for 3; FP32 would spill 94 registers), else 2
 template <typename T, int ENGINE> struct EbOcc { static constexpr int value = 2; };
@@ -799,9 +905,6 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
     int nst = 0;
     typedef __attribute__((address_space(3))) unsigned char lds_u8;
     lds_u8 *ast = (lds_u8 *) (stg0 + (p.sym ? (size_t) NUM_WAVES * BT * LD : 0));
-    // fused update: A's block columns of this row in LDS, alpha and beta
-    typedef __attribute__((address_space(3))) int lds_int;
-    lds_int *acol = (lds_int *) ((unsigned char *) kbits + p.acol_off);
     const int nAr = p.An[ib];
     // fused: this lane's |X - X^2|^2, and the next iterate's sum |U_ij|^2 and
     // trace over the kept blocks (the next iteration's tr X^2 and tr X)
@@ -809,7 +912,6 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
     if (p.fuse) {
         alpha = p.ab[0];
         beta = p.ab[1];
-        for (int q = threadIdx.x; q < nAr; q += 64 * NUM_WAVES) acol[q] = p.Ai[(size_t) ib * p.MA + q];
     }
     if constexpr (Acc::kPipelined && Acc::kStage) {
         using TA = typename Acc::TA;
@@ -875,123 +977,20 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
             }
             return;
         }
-        // sym: the tile at (ib, s) and its transpose at (kb, s')
-        const int sp = kb != ib ? mirror_slot(p, mp, kb, ib) : -1;
-        auto wave_sync = [&]() {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        };
-        bool kept = keep;
-        if (p.fuse) {
-            // U = alpha X[ib, kb] + beta Y, Y the product's block when the x2
-            // rule keeps it (else 0), formed in the staging tile; U kept iff
-            // it is the diagonal block or max |U| > thr (the add's rule;
-            // every X block is reached through its row's diagonal block, so
-            // none is left out); |X - Y|^2 counted twice off the diagonal
-            // (the mirror block)
-            acc.store(stg, LD);
-            wave_sync();
-            if (kb == ib) {  // the diagonal block takes its upper triangle
-                for (int e = lane; e < (int) B2; e += 64) {
-                    const int r = e / BT, c = e % BT;
-                    if (r > c) stg[r * LD + c] = E::conj(stg[c * LD + r]);
-                }
-                wave_sync();
-            }
-            int jx = -1;
-            for (int c0 = 0; c0 < nAr; c0 += 64) {
-                const uint64_t b = ballot64(c0 + lane < nAr && acol[c0 + lane] == kb);
-                if (b) {
-                    jx = c0 + __ffsll((unsigned long long) b) - 1;
-                    break;
-                }
-            }
-            // X's block in chunks of a lane's elements (all of them for 4-byte
-            // elements, two at a time for 8-byte ones, whose kernel has no
-            // registers to spare), each chunk's loads issued before any is
-            // used (from the LDS stage when it holds the exact tile)
-            constexpr int QE = (int) (B2 / 64);
-            static_assert(B2 % 64 == 0, "a tile is whole rows of 64 lanes");
-            constexpr int CH = sizeof(T) <= 4 ? QE : (QE >= 2 ? 2 : QE);
-            bool staged = false;
+        // X's block from the LDS stage when it holds the exact tile
+        auto xl = [&](int jx, int e) -> T {
             if constexpr (Acc::kStage) {
                 using TA = typename Acc::TA;
-                if constexpr (std::is_same<TA, T>::value) staged = jx >= 0 && jx < nst;
-            }
-            const T *xg = Av + ((size_t) ib * p.MA + (jx >= 0 ? jx : 0)) * B2;
-            double mu = 0.0, dn = 0.0, fu = 0.0, tu = 0.0;
-#pragma unroll 1
-            for (int q0 = 0; q0 < QE; q0 += CH) {
-                T xv[CH];
-#pragma unroll
-                for (int j = 0; j < CH; j++) {
-                    const int e = lane + 64 * (q0 + j);
-                    xv[j] = E::zero();
-                    if constexpr (Acc::kStage) {
-                        using TA = typename Acc::TA;
-                        if constexpr (std::is_same<TA, T>::value) {
-                            constexpr int TE = 16 / (int) sizeof(TA);
-                            const int r = e / BT, c = e % BT;
-                            if (staged)
-                                xv[j] = *((lds_ptr<TA>) ast + jx * (int) B2 + r * BT +
-                                          Acc::swz(r, c / TE) * TE + c % TE);
-                        }
-                    }
-                    if (!staged && jx >= 0) xv[j] = xg[e];
-                }
-#pragma unroll
-                for (int j = 0; j < CH; j++) {
-                    const int e = lane + 64 * (q0 + j), r = e / BT, c = e % BT;
-                    const T y = keep ? stg[r * LD + c] : E::zero();
-                    const T u = E::axpy(E::axpy(E::zero(), alpha, xv[j]), beta, y);
-                    stg[r * LD + c] = u;
-                    mu = fmax(mu, E::mag(u));
-                    dn += E::abs2(E::sub(xv[j], y));
-                    fu += E::abs2(u);
-                    if (r == c) tu += E::re(u);
-                }
-            }
-            nrm_l += kb == ib ? dn : 2.0 * dn;
-            kept = kb == ib || wave_max(mu) > p.thr;
-            if (kept && (s < p.MC || (sp >= 0 && sp < p.MC))) {
-                frob_l += kb == ib ? fu : 2.0 * fu;
-                if (kb == ib) trn_l += tu;
-            }
-            wave_sync();
-        }
-        if (lane == 0) {
-            p.kflag[(size_t) ib * p.maxs + s] = kept;
-            if (sp >= 0) p.kflag[(size_t) kb * p.maxs + sp] = kept;
-        }
-        if (kept && (s < p.MC || (sp >= 0 && sp < p.MC))) {
-            if (!p.fuse) {
-                acc.store(stg, LD);
-                wave_sync();
-            }
-            if (s < p.MC) {
-                const size_t sc = (size_t) ib * p.MC + s;
-                T *D = Cv + sc * B2;
-                for (int e = lane; e < (int) B2; e += 64) {
+                if constexpr (std::is_same<TA, T>::value) {
+                    constexpr int TE = 16 / (int) sizeof(TA);
                     const int r = e / BT, c = e % BT;
-                    D[e] = (kb == ib && r > c) ? E::conj(stg[c * LD + r]) : stg[r * LD + c];
+                    if (jx < nst)
+                        return *((lds_ptr<TA>) ast + jx * (int) B2 + r * BT + Acc::swz(r, c / TE) * TE + c % TE);
                 }
-                if (lane == 0) p.Ci[sc] = kb;
             }
-            if (sp >= 0 && sp < p.MC) {
-                const size_t sc = (size_t) kb * p.MC + sp;
-                T *D = Cv + sc * B2;
-                for (int e = lane; e < (int) B2; e += 64) {
-                    const int r = e / BT, c = e % BT;
-                    D[e] = E::conj(stg[c * LD + r]);
-                }
-                if (lane == 0) p.Ci[sc] = ib;
-            }
-            // the staging tile is read before the next slot overwrites it
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        }
+            return Av[((size_t) ib * p.MA + jx) * B2 + e];
+        };
+        finish_sym<T, BT>(p, acc, ib, s, kb, mp, stg, keep, nAr, alpha, beta, nrm_l, frob_l, trn_l, xl);
     };
     if constexpr (Acc::kPipelined) {
         // One stream of pairs per wavefront.  It claims batches (about
@@ -1035,8 +1034,8 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
                     if (lane == 0) k = atomicAdd(&next_s, 1);
                     k = __shfl(k, 0, 64);
                     if (k >= nbatch) return false;
-                    n.t0 = off[bf[k]];
-                    n.te = off[bf[k + 1]];
+                    n.t0 = bf[k];
+                    n.te = bf[k + 1];
                     if (n.te > n.t0) break;
                 }
             }
@@ -1164,6 +1163,283 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
             p.rowtr[ib] = E::re(tx);
             p.rowtr[p.NB + ib] = t2;
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// numeric pass, double real on the matrix cores (MfmaAccF64)
+//
+// What bounds it is the L2 misses of the tiles: 16 KB per pair of tiles, and
+// few tiles are met twice by one workgroup.  With a workgroup per block row
+// (the FP32 and bf16 kernel above) 64 rows were at work on an XCD at a time
+// and 78% of the reads missed its L2, 16 GB at 7 TB/s for the general X^2 of
+// the 16x16x8-site, 32-orbital lattice (1.25 M pairs).  Here workgroups stay
+// for the whole product and their wavefronts take batches (about STREAM_BATCH
+// pairs, whole slots of one block row) from 8 queues, one per XCD, each an
+// eighth of all batches in block row order: 3 to 7 rows are at work on an
+// XCD, their left tiles stay in its L2, and 45% of the reads miss.  A
+// wavefront whose queue is empty goes on to the next one, so no CU waits for
+// the longest row.  That product: 2.27 -> 1.75 ms with its compaction at
+// 0.11 (matrix cores busy 1.2 ms); the fused symmetric update of the
+// 8x8x6-site lattice (384 block rows, 125 k pairs): 325 -> 240 us.
+//
+// Batches of 8 pairs: the X^2 2.13 ms, the 25 updates of an SP2 loop on the
+// 8x8x6 lattice 7.5 ms; of 16, 2.13 and 7.9; of 32, 2.24 and 8.3; of 4, 2.20
+// and 7.7.  A wavefront's first batch is its own number, not a claim, and a
+// workgroup asks no queue that it has found empty: 2048 wavefronts that each
+// asked all 8 heads spent 150 us of the update on those atomics.  Three
+// workgroups per CU spill and miss more (2.97 ms), one leaves the matrix
+// cores idle between the pairs of a wavefront (2.48).
+constexpr int EB_GROUPS = 2048;  // groups of block rows in the LDS prefix of batch counts
+
+template <bool SYM>
+__global__ __launch_bounds__(64 * NUM_WAVES, 2) void k_eb_stream(EbParams p) {
+    using T = double;
+    using E = Elem<T>;
+    using Acc = MfmaAccF64;
+    using Frag = Acc::Frag;
+    constexpr int BT = 32;
+    constexpr size_t B2 = (size_t) BT * BT;
+    constexpr int LD = BT + 1;
+    // dynamic LDS: the wavefronts' turned tiles, then (sym) their staging tiles
+    extern __shared__ __align__(16) double smem[];
+    __shared__ int pre[EB_GROUPS + 1];  // batches before each group of rows
+    __shared__ int wsum[NUM_WAVES];
+    __shared__ volatile int empty_s[EB_QUEUES];  // queues found empty
+    __shared__ T diag_s[NUM_WAVES][BT];
+    __shared__ double fz_s[3][NUM_WAVES];
+    if (p.skip && *p.skip) return;
+    const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const T *Av = (const T *) p.Av;
+    const T *Bv = (const T *) p.Bv;
+    T *Cv = (T *) p.Cv;
+    T *stg = smem + (size_t) w * BT * LD;
+    lds_tile turn = (lds_tile) stg;
+    const int gs = (p.NB + EB_GROUPS - 1) / EB_GROUPS;  // rows per group
+    {
+        constexpr int PT = EB_GROUPS / (64 * NUM_WAVES);
+        int v[PT], t = 0;
+#pragma unroll
+        for (int j = 0; j < PT; j++) {
+            const long long r0 = (long long) ((int) threadIdx.x * PT + j) * gs;
+            v[j] = 0;
+            for (int r = 0; r < gs; r++)
+                if (r0 + r < p.NB) v[j] += p.nbat[r0 + r];
+            t += v[j];
+        }
+        int inc = t;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += o;
+        }
+        if (lane == 63) wsum[w] = inc;
+        if (threadIdx.x < EB_QUEUES) empty_s[threadIdx.x] = 0;
+        __syncthreads();
+        int at = inc - t;
+        for (int k = 0; k < w; k++) at += wsum[k];
+#pragma unroll
+        for (int j = 0; j < PT; j++) {
+            pre[threadIdx.x * PT + j] = at;
+            at += v[j];
+        }
+        if (threadIdx.x == 64 * NUM_WAVES - 1) pre[EB_GROUPS] = at;
+        __syncthreads();
+    }
+    const long long total = pre[EB_GROUPS];
+    double alpha = 0.0, beta = 0.0, nrm_l = 0.0, frob_l = 0.0, trn_l = 0.0;
+    if (SYM && p.fuse) {
+        alpha = p.ab[0];
+        beta = p.ab[1];
+    }
+
+    // A unit is up to 64 pairs of a batch; lane q holds pair q's A tile, B
+    // tile, slot and block column.  The unit after the one at work is fetched
+    // one stage per pair (advance), each stage using what the one before
+    // asked for, so that no wait of this chain of five loads stands alone.
+    struct Unit {
+        int ib, np, nA;
+        int sa, bt, sid, kb;  // per lane
+    };
+    enum { CLAIM, FIND, RANGE, PAIRS, TILES, READY, DONE };
+    Unit nu;
+    int stage = FIND, queue = (int) blockIdx.x % EB_QUEUES;
+    int head = (int) blockIdx.x / EB_QUEUES * NUM_WAVES + w, ta = 0, te = 0, b0 = 0, b1 = 0, pv = 0, ja = 0;
+    auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    auto advance = [&]() {
+        if (stage == CLAIM) {
+            // the first queue from this one on that no wavefront of the
+            // workgroup has found empty
+            const uint64_t open = ballot64(lane < EB_QUEUES && !empty_s[(queue + lane) % EB_QUEUES]);
+            if (!open) {
+                stage = DONE;
+                return;
+            }
+            queue = (queue + __ffsll((unsigned long long) open) - 1) % EB_QUEUES;
+            if (lane == 0) head = atomicAdd(&p.nbat[p.NB + queue * EB_HEAD], 1);
+            stage = FIND;
+        } else if (stage == FIND) {
+            const int lo = (int) (total * queue / EB_QUEUES), hi = (int) (total * (queue + 1) / EB_QUEUES);
+            const int h = uni(head);
+            if (h >= hi - lo) {
+                if (lane == 0) empty_s[queue] = 1;
+                stage = CLAIM;
+                return;
+            }
+            // the group of rows that holds batch `it`, by 64 bounds, then 32
+            const int it = lo + h;
+            constexpr int F = EB_GROUPS / 64;
+            const int cb = popc64(ballot64(pre[(lane + 1) * F] <= it));
+            const int fb = popc64(ballot64(lane < F && pre[cb * F + (lane < F ? lane : 0) + 1] <= it));
+            int rem = it - uni(pre[cb * F + fb]);
+            int ib = (cb * F + fb) * gs;
+            for (int nb; gs > 1 && rem >= (nb = uni(p.nbat[ib])); ib++) rem -= nb;
+            nu.ib = ib;
+            const int *bf = p.bfirst + (size_t) ib * (p.maxp / STREAM_BATCH + 2) + rem;
+            b0 = bf[0];
+            b1 = bf[1];
+            nu.nA = p.An[ib];
+            stage = RANGE;
+        } else if (stage == RANGE || stage == PAIRS) {
+            if (stage == RANGE) {
+                ta = uni(b0);
+                te = uni(b1);
+                nu.nA = uni(nu.nA);
+            }
+            if (te <= ta) {
+                stage = CLAIM;
+                return;
+            }
+            nu.np = te - ta < 64 ? te - ta : 64;
+            const size_t t = (size_t) nu.ib * p.maxp + ta + (lane < nu.np ? lane : 0);
+            pv = p.pairs[t];
+            nu.sid = p.pslot[t];
+            ta += nu.np;
+            stage = TILES;
+        } else if (stage == TILES) {
+            nu.sa = nu.ib * p.MA + (int) ((unsigned) pv >> 16);
+            ja = p.Ai[nu.sa];
+            nu.kb = p.skb[(size_t) nu.ib * p.maxs + nu.sid];
+            stage = READY;
+        }
+    };
+    auto next_ready = [&]() -> bool {
+        while (stage < READY) advance();
+        return stage == READY;
+    };
+    auto take = [&](Unit &u) {
+        nu.bt = ja * p.MB + (pv & 0xffff);
+        u = nu;
+        stage = ta < te ? PAIRS : CLAIM;
+    };
+    auto ld = [&](int sa, int bt, Frag &f) { Acc::load(Av + (size_t) sa * B2, Bv + (size_t) bt * B2, f); };
+    auto pick = [](int v, int q) { return __builtin_amdgcn_readlane(v, q); };
+    auto fence = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // keep rule, traces and the stores of slot s's finished tile
+    auto finish = [&](const Acc &acc, int ib, int s, int kb, int nA, const MirrorProbe &mp) {
+        const double nrm = wave_max(acc.maxmag());
+        const bool keep = kb == ib || nrm > p.thr;
+        if (p.kind == 0 && !p.fuse && kb == ib) {
+            // tr X and tr X^2 of the row: the diagonals of the two diagonal
+            // blocks, each summed in order
+            const int bi = p.bsize[ib];
+            int jd = -1;
+            for (int c0 = 0; c0 < nA && jd < 0; c0 += 64) {
+                const uint64_t b =
+                    ballot64(c0 + lane < nA && p.Ai[(size_t) ib * p.MA + (c0 + lane < nA ? c0 + lane : 0)] == ib);
+                if (b) jd = c0 + __ffsll((unsigned long long) b) - 1;
+            }
+            acc.diag(diag_s[w]);
+            fence();
+            if (lane == 0) {
+                double t = 0.0;
+                for (int kk = 0; kk < bi; kk++) t += diag_s[w][kk];
+                p.rowtr[p.NB + ib] = t;
+            }
+            fence();
+            if (jd >= 0) {
+                if (lane < bi) diag_s[w][lane] = Av[((size_t) ib * p.MA + jd) * B2 + lane * (BT + 1)];
+                fence();
+                if (lane == 0) {
+                    double t = 0.0;
+                    for (int kk = 0; kk < bi; kk++) t += diag_s[w][kk];
+                    p.rowtr[ib] = t;
+                }
+                fence();
+            }
+        }
+        if constexpr (SYM) {
+            auto xl = [&](int jx, int e) -> T { return Av[((size_t) ib * p.MA + jx) * B2 + e]; };
+            finish_sym<T, BT>(p, acc, ib, s, kb, mp, stg, keep, nA, alpha, beta, nrm_l, frob_l, trn_l, xl);
+        } else {
+            if (lane == 0) p.kflag[(size_t) ib * p.maxs + s] = keep;
+            if (keep && s < p.MC) {
+                const size_t sc = (size_t) ib * p.MC + s;
+                acc.store(Cv + sc * B2);
+                if (lane == 0) p.Ci[sc] = kb;
+            }
+        }
+    };
+    if (next_ready()) {
+        Unit cu;
+        take(cu);
+        Acc acc;
+        acc.zero();
+        Frag f;
+        int q = 0;
+        bool first = true;  // of its slot
+        MirrorProbe mp;
+        ld(pick(cu.sa, 0), pick(cu.bt, 0), f);
+        while (true) {
+            // pair q of cu: its left tile goes to LDS, its right tile to rt,
+            // and the pair after it loads into f while the products run
+            Acc::put(turn, f);
+            doublex2 rt[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) rt[k] = f.r[k];
+            fence();
+            const int slot = pick(cu.sid, q), kb = pick(cu.kb, q), ib = cu.ib, nA = cu.nA;
+            if (SYM && first && kb != ib) mp = mirror_probe(p, kb);
+            bool more = true;
+            if (q + 1 < cu.np) {
+                if (stage < READY) advance();
+                q++;
+            } else if (next_ready()) {
+                take(cu);
+                q = 0;
+            } else {
+                more = false;
+            }
+            if (more) ld(pick(cu.sa, q), pick(cu.bt, q), f);
+            acc.mma(turn, rt);
+            fence();
+            first = !more || pick(cu.sid, q) != slot || cu.ib != ib;
+            if (first) {
+                finish(acc, ib, slot, kb, nA, mp);
+                acc.zero();
+            }
+            if (!more) break;
+        }
+    }
+    if (!SYM || !p.fuse) return;
+    for (int off = 32; off > 0; off >>= 1) {
+        nrm_l += __shfl_xor(nrm_l, off, 64);
+        frob_l += __shfl_xor(frob_l, off, 64);
+        trn_l += __shfl_xor(trn_l, off, 64);
+    }
+    if (lane == 0) {
+        fz_s[0][w] = trn_l;
+        fz_s[1][w] = frob_l;
+        fz_s[2][w] = nrm_l;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        double t = 0.0;
+        for (int v = 0; v < NUM_WAVES; v++) t += fz_s[threadIdx.x][v];
+        p.rownorm[(size_t) threadIdx.x * gridDim.x + blockIdx.x] = t;
     }
 }
 
@@ -1564,9 +1840,10 @@ __global__ __launch_bounds__(256) void k_eb_trace_frob(int NB, int MB, const T *
     }
 }
 
-// the fused SP2 product's three per-row sums (next tr X, next tr X^2, and
-// |X - X^2|^2) into status scalars 0, 1, 2: one block of 1024 threads, each
-// sum over a fixed partition and a fixed tree (one launch, not three)
+// the fused SP2 product's three sums over its block rows or workgroups (next
+// tr X, next tr X^2, and |X - X^2|^2) into status scalars 0, 1, 2: one block
+// of 1024 threads, each sum over a fixed partition and a fixed tree (one
+// launch, not three)
 __global__ __launch_bounds__(1024) void k_eb_sum3(const double *x, int n, bmlhip_status *st,
                                                   const int *skip) {
     __shared__ double part[1024];
@@ -1685,10 +1962,22 @@ int report(const char *what) {
     return fail_msg(3, "%s: %s", what, hipGetErrorString(e));
 }
 
+template <typename T, int BT>
+int launch_compact(const EbParams &p, hipStream_t s) {
+    const int nbits = p.maxs < p.MC ? p.maxs : p.MC;
+    const size_t lc = 2 * sizeof(int) * (size_t) (nbits + 1);  // the move list
+    if (lc > 64 * 1024) {
+        if (lc > 160 * 1024) return fail_msg(5, "ellblock product: %d block slots per row exceed LDS", p.MC);
+        (void) hipFuncSetAttribute((const void *) k_eb_compact<T, BT>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int) lc);
+    }
+    hipLaunchKernelGGL((k_eb_compact<T, BT>), dim3(p.NB), dim3(64), lc, s, p);
+    return report("k_eb_compact");
+}
+
 template <typename T, int ENGINE, int BT>
 int launch_numeric(const EbParams &p, hipStream_t s) {
-    if constexpr (ENGINE != 0 && !(BT == 32 && (std::is_same<T, float>::value ||
-                                                (ENGINE == 1 && std::is_same<T, double>::value)))) {
+    if constexpr (ENGINE != 0 && !(BT == 32 && std::is_same<T, float>::value)) {
         return fail_msg(2, "no MFMA engine for this element type and tile");
     } else {
         // kept flags, then (sym) a staging tile per wavefront, as the kernel
@@ -1699,8 +1988,6 @@ int launch_numeric(const EbParams &p, hipStream_t s) {
         if (lds > 160 * 1024) return fail_msg(5, "ellblock product: %d block slots per row exceed LDS", p.MC);
         EbParams q = p;
         q.ka = 0;
-        // fused update: A's block columns after the A tiles
-        const size_t acol_bytes = p.fuse ? ((size_t) p.MA * sizeof(int) + 15) / 16 * 16 : 0;
         if (AccOf<T, ENGINE, BT>::type::kStage) {
             // A tiles staged in LDS: as many as fit in the block's share of a
             // CU's LDS, at most the row width.  Default share: 78 KB (two
@@ -1717,33 +2004,39 @@ int launch_numeric(const EbParams &p, hipStream_t s) {
             }
             const long share = budget > 0 ? budget : 1024L * (ENGINE == 2 ? 48 : 78);
             const long b = share < 156L * 1024 ? share : 156L * 1024;
-            const long used = (long) (lds + acol_bytes);
-            long ka = b > used ? (b - used) / (long) tb : 0;
+            long ka = b > (long) lds ? (b - (long) lds) / (long) tb : 0;
             if (ka > cap) ka = cap;
             if (ka > p.MA) ka = p.MA;
             q.ka = (int) ka;
             lds += (size_t) ka * tb;
         }
-        q.acol_off = (int) lds;
-        lds += acol_bytes;
-        if (lds > 160 * 1024) return fail_msg(5, "ellblock product: %d block slots per row exceed LDS", p.MA);
         if (lds > 64 * 1024)
             (void) hipFuncSetAttribute((const void *) k_eb_numeric<T, ENGINE, BT>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
         hipLaunchKernelGGL((k_eb_numeric<T, ENGINE, BT>), dim3(p.NB), dim3(64 * NUM_WAVES), lds, s,
                            q);
         int rc = report("k_eb_numeric");
-        if (rc || !p.sym) return rc;
-        const int nbits = p.maxs < p.MC ? p.maxs : p.MC;
-        const size_t lc = 2 * sizeof(int) * (size_t) (nbits + 1);  // the move list
-        if (lc > 64 * 1024) {
-            if (lc > 160 * 1024) return fail_msg(5, "ellblock product: %d block slots per row exceed LDS", p.MC);
-            (void) hipFuncSetAttribute((const void *) k_eb_compact<T, BT>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int) lc);
-        }
-        hipLaunchKernelGGL((k_eb_compact<T, BT>), dim3(p.NB), dim3(64), lc, s, p);
-        return report("k_eb_compact");
+        return rc || !p.sym ? rc : launch_compact<T, BT>(p, s);
     }
+}
+
+// workgroups of k_eb_stream: two on every CU
+int stream_groups() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    return (2 * cus + EB_QUEUES - 1) / EB_QUEUES * EB_QUEUES;
+}
+
+int launch_stream(const EbParams &p, int groups, hipStream_t s) {
+    const size_t lds = sizeof(double) * (size_t) NUM_WAVES * 32 * 33;
+    if (p.sym)
+        hipLaunchKernelGGL(k_eb_stream<true>, dim3(groups), dim3(64 * NUM_WAVES), lds, s, p);
+    else
+        hipLaunchKernelGGL(k_eb_stream<false>, dim3(groups), dim3(64 * NUM_WAVES), lds, s, p);
+    int rc = report("k_eb_stream");
+    return rc ? rc : launch_compact<double, 32>(p, s);
 }
 
 template <typename T>
@@ -1796,7 +2089,13 @@ int eb_product_typed(const bmlhip_eb_args *a) {
     p.maxs = (int) maxs;
     p.maxp = (int) maxp;
     const size_t NB = (size_t) a->NB;
-    p.rowtr = (double *) bmlhip_scratch(0, sizeof(double) * 3 * (NB + 1));
+    // FP64 products on the matrix cores run in k_eb_stream
+    const bool stream = std::is_same<T, double>::value && a->bt == 32 && a->engine == 1;
+    const int groups = stream ? stream_groups() : a->NB;
+    const size_t nsum = NB > (size_t) groups ? NB : (size_t) groups;
+    p.batch = stream ? STREAM_BATCH : EB_BATCH;
+    p.head0 = groups / EB_QUEUES * NUM_WAVES;
+    p.rowtr = (double *) bmlhip_scratch(0, sizeof(double) * 3 * (nsum + 1));
     // fused update: the next iterate's traces, then the rows' norms
     p.rownorm = p.rowtr;
     p.cnt = (int *) bmlhip_scratch(3, sizeof(int) * (NB + 1));
@@ -1804,14 +2103,15 @@ int eb_product_typed(const bmlhip_eb_args *a) {
     p.soff = (int *) bmlhip_scratch(5, sizeof(int) * (NB * (maxs + 1) + 1));
     p.pairs = (int *) bmlhip_scratch(6, sizeof(int) * (NB * maxp + 1));
     p.pslot = (int *) bmlhip_scratch(10, sizeof(int) * (NB * maxp + 1));
-    p.bfirst = (int *) bmlhip_scratch(11, sizeof(int) * (NB * (maxp / EB_BATCH + 2) + 1));
+    p.bfirst = (int *) bmlhip_scratch(11, sizeof(int) * (NB * (maxp / p.batch + 2) + NB + EB_QUEUES * EB_HEAD));
+    p.nbat = p.bfirst ? p.bfirst + NB * (maxp / p.batch + 2) : nullptr;
     if ((long long) a->NB * a->MA >= (1ll << 31) || (long long) a->NB * a->MB >= (1ll << 31))
         return fail_msg(5, "ellblock product: more than 2^31 block slots");
     p.sym = a->kind == 0 && a->sym && a->engine != 0;
     p.fuse = p.sym && a->fuse;
     p.ab = a->d_ab;
     if (p.fuse && !p.ab) return fail_msg(2, "ellblock product: the fused update needs alpha, beta");
-    if (p.sym && !(p.kflag = (int *) bmlhip_scratch(1, sizeof(int) * (NB * maxs + 1))))
+    if ((p.sym || stream) && !(p.kflag = (int *) bmlhip_scratch(1, sizeof(int) * (NB * maxs + 1))))
         return fail_msg(4, "ellblock product: scratch allocation failed");
     p.rowstat = (int4 *) bmlhip_scratch(BMLHIP_ROWSTAT_SLOT, sizeof(int4) * (NB + 1));
     if (!p.rowtr || !p.cnt || !p.skb || !p.soff || !p.pairs || !p.pslot || !p.bfirst || !p.rowstat)
@@ -1852,7 +2152,7 @@ int eb_product_typed(const bmlhip_eb_args *a) {
     } else if (std::is_same<T, float>::value && a->bt == 32 && a->engine == 2) {
         rc = launch_numeric<T, 2, 32>(p, s);
     } else if (std::is_same<T, double>::value && a->bt == 32 && a->engine == 1) {
-        rc = launch_numeric<T, 1, 32>(p, s);
+        rc = launch_stream(p, groups, s);
     } else {
         switch (a->bt) {
         case 8: rc = launch_numeric<T, 0, 8>(p, s); break;
@@ -1870,7 +2170,7 @@ int eb_product_typed(const bmlhip_eb_args *a) {
     if (p.fuse) {
         // the rows' |X - X^2|^2, and the next iterate's traces for the next
         // branch decision
-        hipLaunchKernelGGL(k_eb_sum3, dim3(1), dim3(1024), 0, s, p.rownorm, a->NB, p.st, p.skip);
+        hipLaunchKernelGGL(k_eb_sum3, dim3(1), dim3(1024), 0, s, p.rownorm, groups, p.st, p.skip);
         return report("k_eb_sum3");
     }
     if (a->kind == 0) {
