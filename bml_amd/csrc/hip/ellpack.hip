@@ -1121,22 +1121,39 @@ __device__ __forceinline__ void pk_get(const unsigned *P, size_t e, T &v, int &c
     v = cv.t;
     c = (int) x.w[NW - 1];
 }
-// Entry k of a packed row starting at Pj: a scalar base and a 32-bit
-// per-lane byte offset (one global load with a scalar address; rows hold
-// fewer than 2^24 entries).
-template <typename T>
-__device__ __forceinline__ void pk_get_at(const unsigned *Pj, unsigned k, T &v, int &c) {
+// Entries lane, lane + 64, ... (n of them) of a packed segment that starts at
+// Pj and holds `left` entries (both uniform): buffer loads, which give zeros
+// past the segment's end.
+template <typename T, int n>
+__device__ __forceinline__ void pk_load(const unsigned *Pj, int left, int lane, T (&v)[n], int (&c)[n]) {
     constexpr int NW = PkW<T>::n;
-    const unsigned off = __umul24(k, 4u * NW);
-    const Words<NW> x = *reinterpret_cast<const Words<NW> *>((const char *) Pj + off);
-    union {
-        T t;
-        unsigned u[NW - 1];
-    } cv;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned *>(Pj), 0, left * (4 * NW), 0x00027000);
 #pragma unroll
-    for (int q = 0; q < NW - 1; q++) cv.u[q] = x.w[q];
-    v = cv.t;
-    c = (int) x.w[NW - 1];
+    for (int u = 0; u < n; u++) {
+        const int off = (lane + 64 * u) * (4 * NW);
+        union {
+            T t;
+            unsigned w[NW - 1];
+        } x;
+        if constexpr (NW == 2) {
+            const auto q = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0);
+            x.w[0] = q[0];
+            c[u] = (int) q[1];
+        } else if constexpr (NW == 3) {
+            const auto q = __builtin_amdgcn_raw_buffer_load_b96(rs, off, 0, 0);
+            x.w[0] = q[0];
+            x.w[1] = q[1];
+            c[u] = (int) q[2];
+        } else {
+            static_assert(NW == 5, "entry of 2, 3 or 5 words");
+            const auto q = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) x.w[k] = q[k];
+            c[u] = (int) __builtin_amdgcn_raw_buffer_load_b32(rs, off + 16, 0, 0);
+        }
+        v[u] = x.t;
+    }
 }
 template <typename T>
 __device__ __forceinline__ int pk_col(const unsigned *P, size_t e) {
@@ -1193,11 +1210,19 @@ struct WinParams {
 };
 
 // Pack pass: one wavefront per row.  Row j's entries are grouped by window
-// (counted, scanned, scattered with LDS counters; the order within a window
-// is the arrival order), boff[j][c] is the first entry of window c,
-// boff[j][nwin] the row length, wmask[j] the windows with entries.  With
-// rowtr the row's tr X (its diagonal) and sum |X_jk|^2 partials are written
-// too.
+// (counted, scanned, scattered with LDS counters), boff[j][c] is the first
+// entry of window c, boff[j][nwin] the row length, wmask[j] the windows with
+// entries.  With rowtr the row's tr X (its diagonal) and sum |X_jk|^2
+// partials are written too.
+//
+// Order within a window: the first entries of the 16 column classes mod 16,
+// then their second entries, and so on.  A 64-bit LDS atomic serves 16 lanes
+// a clock, one from each of 16 bank pairs, so 16 consecutive entries of a
+// segment, which the products add in 16 consecutive lanes, should lie in 16
+// classes; entries in column order put three of them in one on average.  On
+// a two-iteration SP2 of the 24^3 lattice (FP32, ~2600 entries a row) that
+// halved the product's bank conflicts (3.2e9 to 1.6e9 cycles of 6.2e9 to
+// 4.7e9 active), at 0.02 ms more for the pack.
 template <typename T>
 __global__ __launch_bounds__(256) void k_win_pack(int N, int M, const T *Xv, const int *Xi,
                                                   const int *Xn, int MP, int nwin, int wb,
@@ -1205,19 +1230,22 @@ __global__ __launch_bounds__(256) void k_win_pack(int N, int M, const T *Xv, con
                                                   unsigned long long *wmask, double *rowtr,
                                                   double *rowmax, const int *skip,
                                                   const int *row_sys, const int *sys_done) {
-    __shared__ int cnt[4][65];
+    // per window and class: the entries (low 16 bits: at most 2^wb / 16 <= 512)
+    // and those placed so far (high 16 bits)
+    __shared__ __align__(16) unsigned cls[4][64][16];
+    __shared__ int base[4][64];
     if (skip && *skip) return;  // uniform
     const int w = threadIdx.x / 64, lane = threadIdx.x & 63;
     const int j = blockIdx.x * 4 + w;
     const bool live = j < N && !(row_sys && sys_done[row_sys[j]]);
     const int n = live ? Xn[j] : 0;
     const size_t rowX = live ? (size_t) j * M : 0;
-    cnt[w][lane] = 0;
+    for (int e = lane; e < 64 * 16; e += 64) cls[w][e >> 4][e & 15] = 0u;
     __syncthreads();
     double trx = 0.0, sq = 0.0, mx = 0.0;
     for (int e = lane; e < n; e += 64) {
         const int c = Xi[rowX + e];
-        atomicAdd(&cnt[w][c >> wb], 1);
+        atomicAdd(&cls[w][c >> wb][c & 15], 1u);
         if (rowtr || rowmax) {
             const T v = Xv[rowX + e];
             if (c == j) trx += Elem<T>::re(v);
@@ -1230,7 +1258,9 @@ __global__ __launch_bounds__(256) void k_win_pack(int N, int M, const T *Xv, con
         if (lane == 0) rowmax[j] = mx;
     }
     __syncthreads();
-    const int x = lane < nwin ? cnt[w][lane] : 0;
+    int x = 0;
+    if (lane < nwin)
+        for (int q = 0; q < 16; q++) x += (int) cls[w][lane][q];
     int inc = x;
     for (int d = 1; d < 64; d <<= 1) {
         const int o = __shfl_up(inc, d, 64);
@@ -1238,7 +1268,7 @@ __global__ __launch_bounds__(256) void k_win_pack(int N, int M, const T *Xv, con
     }
     const unsigned long long m = ballot64(x > 0);
     __syncthreads();
-    cnt[w][lane] = inc - x;  // next free position of window `lane`
+    base[w][lane] = inc - x;  // first position of window `lane`
     if (live) {
         int *bo = boff + (size_t) j * (nwin + 1);
         if (lane < nwin) bo[lane] = inc - x;
@@ -1252,7 +1282,21 @@ __global__ __launch_bounds__(256) void k_win_pack(int N, int M, const T *Xv, con
     for (int e = lane; e < n; e += 64) {
         const int c = Xi[rowX + e];
         const T v = Xv[rowX + e];
-        const int pos = atomicAdd(&cnt[w][c >> wb], 1);
+        const int cw = c >> wb, cq = c & 15;
+        // the t-th entry of its class: after t entries of every class and the
+        // t-th of the classes below its own, as far as they have them
+        const unsigned t = atomicAdd(&cls[w][cw][cq], 1u << 16) >> 16;
+        unsigned pos = (unsigned) base[w][cw];
+#pragma unroll
+        for (int q4 = 0; q4 < 16; q4 += 4) {
+            const uint4 n4 = *reinterpret_cast<const uint4 *>(&cls[w][cw][q4]);
+            const unsigned k4[4] = {n4.x & 0xffffu, n4.y & 0xffffu, n4.z & 0xffffu, n4.w & 0xffffu};
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const unsigned lim = t + (q4 + u < cq ? 1u : 0u);
+                pos += k4[u] < lim ? k4[u] : lim;
+            }
+        }
         pk_put<T>(P, rowP + pos, v, c);
     }
     if (rowtr && live) {
@@ -1848,8 +1892,10 @@ __global__ __launch_bounds__(64 * W, WinbOcc<T>::value) void k_spgemm_winb(WinPa
     const int MC = p.MC;
     T *Cv = (T *) p.Cv;
     int kept[R], distinct[R];  // block-uniform running counts
-    long long prods[R];        // this wavefront's products per row (wave-uniform)
-    long long streamed = 0;    // this wavefront's entries of B read (wave-uniform)
+    // this lane's products per row and entries of B read (one per 64 union
+    // entries a window: at most 2^8 segments of a row's 2^14 entries)
+    int prods[R];
+    int streamed = 0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
         kept[r] = 0;
@@ -1890,109 +1936,116 @@ __global__ __launch_bounds__(64 * W, WinbOcc<T>::value) void k_spgemm_winb(WinPa
             };
             for (int g0 = next_group(); g0 < nU; g0 = next_group()) {
                 const int e = g0 + lane;
-                int jq = 0, lo = 0, hi = 0;
-                unsigned rq = 0;  // rows with a nonzero coefficient
-                V cs[R];          // the coefficients, widened and scaled by 2^E
+                unsigned long long at = 0;  // first entry of the segment
+                // its entries, and below them a bit for each row with a
+                // nonzero coefficient
+                unsigned sq = 0;
+                V cs[R];  // the coefficients, widened and scaled by 2^E
 #pragma unroll
                 for (int r = 0; r < R; r++) cs[r] = fx_scale(F::widen(E::zero()), 0.0);
                 if (e < nU) {
-                    jq = Uj[e];
+                    const int jq = Uj[e];
                     const int *bo = p.boff + (size_t) jq * nw1;
-                    lo = bo[c];
-                    hi = bo[c + 1];
+                    const int lo = bo[c], len = bo[c + 1] - lo;
+                    at = (unsigned long long) jq * p.MP + lo;
+                    streamed += len;
 #pragma unroll
                     for (int r = 0; r < R; r++) {
                         const T t = Uc[(size_t) e * R + r];
                         cs[r] = fx_scale(F::widen(t), sc);
-                        if (E::nonzero(t)) rq |= 1u << r;
+                        if (E::nonzero(t)) {
+                            sq |= 1u << r;
+                            prods[r] += len;
+                        }
                     }
+                    sq |= (unsigned) len << R;
                 }
-                uint64_t todo = ballot64(hi > lo);
+                uint64_t todo = ballot64(sq >> R);
                 if (!todo) continue;
-                // The group's segments as a sequence of rounds of 256
-                // entries (four per lane), software-pipelined: the next
-                // round's loads are issued before the current round's adds.
-                // Segment state is wave-uniform (scalar registers).
-                struct Seg {
-                    const unsigned *Pj;  // row j's packed entries
-                    int l1;              // segment end
-                    unsigned rm;
+                // The group's segments as a sequence of rounds of up to 256
+                // entries (four per lane) of one segment, software-pipelined:
+                // the next round's loads are issued before the current
+                // round's adds.  Segment state is wave-uniform (scalar
+                // registers).  Loads go through a buffer that ends with the
+                // segment: lanes past it read nothing, with no address
+                // arithmetic, and a round that does not exist is loaded from
+                // an empty one, so that the loads are straight-line code and
+                // the adds wait only for their own.  Products are counted per
+                // lane when a group is read, not per segment.  Together 9.7
+                // vector and 10 scalar instructions per wavefront's atomic
+                // came down to 5.5 and 6, and the product of the 24^3
+                // lattice's iterate from 16.8 to 15.1 ms: what is left is
+                // the atomics themselves (about 9 of 11.8 clocks each) and
+                // 103 GB of entries past the L2 at 6.7 TB/s.  8 rows per
+                // block stream 70 GB and take as long (two blocks per CU);
+                // three rounds in flight and windows of 2^11 gain nothing.
+                constexpr int EPL = 4;
+                constexpr unsigned ALL = (1u << R) - 1u;
+                struct Round {
+                    int n;        // entries from the round's first to its segment's end
+                    unsigned rm;  // rows with a nonzero coefficient
                     V a[R];
+                    T v[EPL];
+                    int col[EPL];
                 };
-                auto fetch = [&](Seg &sg, int &kb) {
-                    const int q = __ffsll((long long) todo) - 1;
-                    todo &= todo - 1ull;
-                    const int j = __builtin_amdgcn_readlane(jq, q);
-                    kb = __builtin_amdgcn_readlane(lo, q);
-                    sg.l1 = __builtin_amdgcn_readlane(hi, q);
-                    sg.rm = (unsigned) __builtin_amdgcn_readlane((int) rq, q);
-                    sg.Pj = P + (size_t) j * p.MP * PkW<T>::n;
+                const unsigned *Pj = P;  // the segment at work: its next entry
+                int left = 0;            // and how many are left
+                // the round after `prev`, of the same segment or the next
+                auto next = [&](Round &q, const Round &prev) {
+                    if (left > 0) {
+                        q.rm = prev.rm;
 #pragma unroll
-                    for (int r = 0; r < R; r++) sg.a[r] = bcast<64>(cs[r], q);
-                    const int len = sg.l1 - kb;
-                    streamed += len;
+                        for (int r = 0; r < R; r++) q.a[r] = prev.a[r];
+                    } else if (todo) {
+                        const int l = __ffsll((unsigned long long) todo) - 1;
+                        todo &= todo - 1ull;
+                        const unsigned s0 = (unsigned) __builtin_amdgcn_readlane((int) sq, l);
+                        left = (int) (s0 >> R);
+                        q.rm = s0 & ALL;
+                        Pj = P + bcast<64>(at, l) * PkW<T>::n;
 #pragma unroll
-                    for (int r = 0; r < R; r++)
-                        if (sg.rm >> r & 1u) prods[r] += len;
-                };
-                // EPL loads per lane, always issued (straight-line code, so
-                // that the adds wait only for their own round's loads):
-                // lanes past the segment's end reload its last entry and
-                // mark it column -1.
-                constexpr int EPL = 4;  // 256 entries per round
-                auto load = [&](const Seg &sg, int kb, T (&bv)[EPL], int (&cv)[EPL]) {
-                    const int k0 = kb + lane, kl = sg.l1 - 1;
-#pragma unroll
-                    for (int u = 0; u < EPL; u++) {
-                        const int k = k0 + 64 * u;
-                        pk_get_at<T>(sg.Pj, (unsigned) (k < kl ? k : kl), bv[u], cv[u]);
+                        for (int r = 0; r < R; r++) q.a[r] = bcast<64>(cs[r], l);
                     }
-#pragma unroll
-                    for (int u = 0; u < EPL; u++)
-                        if (k0 + 64 * u > kl) cv[u] = -1;
+                    q.n = left;
+                    pk_load<T, EPL>(Pj, left > 0 ? left : 0, lane, q.v, q.col);
+                    Pj += 64 * EPL * PkW<T>::n;
+                    left -= 64 * EPL;
                 };
-                auto add = [&](const Seg &sg, T bv, int col) {
-                    if (col < 0) return;
-                    const V wv = F::widen(bv);
+                auto use = [&](const Round &q) {
+                    auto entries = [&](auto all) {
+                        constexpr bool EVERY = decltype(all)::value;
 #pragma unroll
-                    for (int r = 0; r < R; r++) {
-                        if (!(sg.rm >> r & 1u)) continue;  // uniform
-                        int sl = r * WC + col;
-                        if constexpr (DIAG && SYM) sl = col >= i0 + r ? sl : dummy + cbase;
-                        fx_add(wc, sl, sg.a[r], wv);
-                        if constexpr (DIAG && !SYM) dtouch[r] = dtouch[r] | (col == i0 + r);
-                    }
+                        for (int u = 0; u < EPL; u++) {
+                            if (64 * u >= q.n) break;  // uniform
+                            if (64 * u + lane < q.n) {
+                                const V wv = F::widen(q.v[u]);
+                                const int col = q.col[u];
+#pragma unroll
+                                for (int r = 0; r < R; r++) {
+                                    if (!EVERY && !(q.rm >> r & 1u)) continue;  // uniform
+                                    int sl = r * WC + col;
+                                    if constexpr (DIAG && SYM) sl = col >= i0 + r ? sl : dummy + cbase;
+                                    fx_add(wc, sl, q.a[r], wv);
+                                    if constexpr (DIAG && !SYM) dtouch[r] = dtouch[r] | (col == i0 + r);
+                                }
+                            }
+                        }
+                    };
+                    if (q.rm == ALL)
+                        entries(std::true_type{});
+                    else
+                        entries(std::false_type{});
                 };
-                Seg cur, nxt;
-                int kc, kn;
-                T bv[EPL], nv[EPL];
-                int cv[EPL], dv[EPL];
-                fetch(cur, kc);
-                load(cur, kc, bv, cv);
+                Round q0, q1;
+                q1.rm = 0;
+                next(q0, q1);
                 while (true) {
-                    // the round after (kc): the rest of this segment, or the next
-                    const bool same = kc + 64 * EPL < cur.l1;
-                    const bool more = same || todo != 0ull;
-                    if (same) {
-                        nxt = cur;
-                        kn = kc + 64 * EPL;
-                    } else if (more) {
-                        fetch(nxt, kn);
-                    } else {
-                        nxt = cur;  // a round that is loaded and never added
-                        kn = kc;
-                    }
-                    load(nxt, kn, nv, dv);
-#pragma unroll
-                    for (int u = 0; u < EPL; u++) add(cur, bv[u], cv[u]);
-                    if (!more) break;
-                    cur = nxt;
-                    kc = kn;
-#pragma unroll
-                    for (int u = 0; u < EPL; u++) {
-                        bv[u] = nv[u];
-                        cv[u] = dv[u];
-                    }
+                    next(q1, q0);
+                    use(q0);
+                    if (q1.n <= 0) break;
+                    next(q0, q1);
+                    use(q1);
+                    if (q0.n <= 0) break;
                 }
             }
         };
@@ -2097,10 +2150,11 @@ __global__ __launch_bounds__(64 * W, WinbOcc<T>::value) void k_spgemm_winb(WinPa
         }
     }
     // row records, traces, norms
-    if (lane == 0) {
 #pragma unroll
-        for (int r = 0; r < R; r++) prods_s[w][r] = prods[r];
-        prods_s[w][R] = streamed;
+    for (int r = 0; r <= R; r++) {
+        long long v = r < R ? prods[r < R ? r : 0] : streamed;
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+        if (lane == 0) prods_s[w][r] = v;
     }
     __syncthreads();
 #pragma unroll
@@ -3136,7 +3190,7 @@ int win_pack(int N, int M, const void *Xv, const int *Xi, const int *Xn, int wbi
     if (nwin < 0)
         return fail_msg(5, "window engine: N=%d needs more than %d windows of 2^%d columns", N,
                         BMLHIP_WIN_MAX_WINDOWS, wbits);
-    if (M >= (1 << 24))  // packed rows are addressed with 24-bit entry offsets
+    if (M >= (1 << 24))  // the limit of a packed row
         return fail_msg(5, "window engine: rows of M=%d entries (at most 2^24 - 1)", M);
     unsigned *P = (unsigned *) bmlhip_scratch(BMLHIP_WIN_PACK_SLOT,
                                               sizeof(unsigned) * PkW<T>::n * ((size_t) N * M + 1));
