@@ -1,5 +1,7 @@
 /*
- * Launch-shape choice for the ELLPACK row-product kernels.
+ * Launch-shape choice for the ELLPACK row-product kernels.  The exact engine
+ * takes the direct-index kernel where its index fits (pick_direct below);
+ * what follows is the hash kernels' choice.
  *
  * group (lanes per output row) follows the length of the rows of B that a
  * step streams: a step holds three GROUP-wide chunks of a row of B in

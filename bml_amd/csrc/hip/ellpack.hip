@@ -1,6 +1,9 @@
-// gfx950 kernels for the ELLPACK-R thresholded multiply path.
+// gfx950 kernels for the ELLPACK-R thresholded multiply path: the hash-table
+// products (the exact engine's direct-index kernel, which takes most
+// products, is rowdir.hip), the unordered and window engines, the adds and
+// the single-pass kernels.
 //
-// Row accumulator.  Every output row is built by a "group" of GROUP lanes
+// Row accumulator of the hash kernels.  Every output row is built by a "group" of GROUP lanes
 // (8..64, so 64/GROUP rows per 64-lane wavefront) that owns an open-addressed
 // hash table in LDS: keys[] (column, -1 = empty), vals[] (the running sum)
 // and ord[] (slot of the r-th distinct column, in first-touch order).  The

@@ -432,7 +432,7 @@ static int batch_alloc(batch_dev *d, int nsys, int N, const char *what)
     d->b.d_rowtr = d->rowtr;
     d->b.d_rownorm = d->rownorm;
     /* The work queue (BML_HIP_BATCH_QUEUE=1) lists the unfinished systems'
-     * rows for persistent hash and add kernels; off, every row has its place
+     * rows for persistent hash kernels; off, every row has its place
      * in a grid and rows of finished systems return at once, which ran
      * faster on every engine (unordered: 147 against 129 solves/s on the
      * 512-system batch) */
