@@ -1782,13 +1782,14 @@ __device__ __forceinline__ cf64 fx_scale(cf64 v, double sc) { return {v.x * sc, 
 
 // Waves per SIMD the compiler is asked to fit (registers).  The fused step's
 // 4-row blocks of 2^10-column windows need 37 KB (float) and 42 KB (double)
-// of LDS, so 3 blocks of 8 wavefronts fit a CU; real types hold their
-// registers to 6 waves per SIMD (some spill to scratch), which ran the
-// 32^3 SP2 step's kernel 1.2x (float) and 1.15x (double) faster than the
-// 4-wave default.  Complex blocks are LDS-bound at 1-2 per CU.
+// of LDS, so 3 blocks of 8 wavefronts fit a CU.  Float holds its registers
+// to 6 waves per SIMD (three blocks).  Double holds them to 4 (two blocks):
+// its 12-byte entries past the L2 are the bound, and three blocks a CU drift
+// further apart in X (437 GB a launch on the 32^3 SP2 step, at 7.2 TB/s) and
+// spill: 61.0 ms at 6, 47.6 at 4.  Complex blocks are LDS-bound at 1-2 per CU.
 template <typename T> struct WinbOcc { static constexpr int value = 1; };
 template <> struct WinbOcc<float> { static constexpr int value = 6; };
-template <> struct WinbOcc<double> { static constexpr int value = 6; };
+template <> struct WinbOcc<double> { static constexpr int value = 4; };
 template <typename T, int W, int WB, int R, bool SYM, bool FUSE>
 __global__ __launch_bounds__(64 * W, WinbOcc<T>::value) void k_spgemm_winb(WinParams p) {
     using E = Elem<T>;
