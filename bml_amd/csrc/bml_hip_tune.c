@@ -532,8 +532,8 @@ void bmlh_tuned_spgemm(int precision, int N, int max_a, int max_b, int touched_h
     } else if (out->engine == BMLHIP_ROW_DIRECT) {
         /* wavefronts per block and the LDS that goes with them */
         const int w0 = best.waves, t0 = best.table;
-        for (int w = w0 / 2; w <= 2 * w0 && w <= 8; w *= 2) {
-            if (w < 1 || w == w0)
+        for (int w = w0 > 1 ? w0 / 2 : 1; w <= 2 * w0 && w <= 8; w *= 2) {
+            if (w == w0)
                 continue;
             c = best;
             c.waves = w;

@@ -1,0 +1,79 @@
+"""The search for a launch shape of the direct-index row product, and the
+shapes it reads back from its cache (host logic, no GPU): the measurement is
+replaced by one that times nothing and notes the candidates."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import pytest
+
+from bml_amd import hip
+
+EXACT, DIRECT = 0, 3  # engines of a launch shape
+SINGLE, DOUBLE, SINGLE_C, DOUBLE_C = 1, 2, 3, 4
+ELEM = {SINGLE: 4, DOUBLE: 8, SINGLE_C: 8, DOUBLE_C: 16}
+SQUARE = 1
+
+
+class Shape(C.Structure):
+    _fields_ = [(n, C.c_int) for n in ("group", "table", "bucket", "remap", "waves", "engine",
+                                       "wbits", "wrows")]
+
+    def key(self):
+        return tuple(getattr(self, n) for n, _ in self._fields_)
+
+
+MEASURE = C.CFUNCTYPE(C.c_int, C.POINTER(Shape), C.c_void_p, C.POINTER(C.c_double))
+
+
+def copy_of(sh):
+    out = Shape()
+    C.pointer(out)[0] = sh
+    return out
+
+
+def search(prec, N, n, touched=0, ms=lambda sh: 1.0):
+    """bmlh_tuned_spgemm for an N x N square of rows of n entries: the shape
+    taken and the candidates measured."""
+    tried = []
+
+    @MEASURE
+    def measure(sh, ctx, out):
+        tried.append(copy_of(sh[0]))
+        out[0] = ms(sh[0])
+        return 0
+
+    out = Shape()
+    hip.lib().bmlh_tuned_spgemm(prec, N, n, n, touched, n if touched else 0, SQUARE, C.byref(out),
+                                measure, None)
+    return out, tried
+
+
+def analytic(prec, N, n, touched=0):
+    out = Shape()
+    hip.lib().bmlh_pick_spgemm(prec, N, N, n, n, touched, n if touched else 0, SQUARE, C.byref(out))
+    return out
+
+
+@pytest.fixture
+def tuner():
+    hip.autotune_clear()
+    hip.set_autotune(True, "")
+    yield
+    hip.set_autotune(False, "")
+    hip.autotune_clear()
+
+
+def test_search_from_one_wavefront_ends():
+    """Shapes of one wavefront (few rows, or long ones) are searched too."""
+    code = ("import test_autotune_direct as t\n"
+            "t.hip.set_autotune(True, '')\n"
+            "for N in (100, 300, 500, 511, 4096):\n"
+            "    t.hip.autotune_clear()\n"
+            "    sh, tried = t.search(t.DOUBLE, N, 33)\n"
+            "    assert sh.engine == t.DIRECT and tried, N\n"
+            "    assert {1, 2} <= {s.waves for s in tried}, N\n")
+    here = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([here, os.path.dirname(here)]))
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=60, env=env)
