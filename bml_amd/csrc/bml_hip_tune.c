@@ -47,9 +47,11 @@
  * more than that forms them in several passes, so a wrong guess costs time
  * only; without a hint the bound min(span, max_a * max_b) is far above the
  * truth, and 3000 columns are the most that are provided for.
- * Rows so short that all columns fit are indexed by the column itself. */
+ * Rows so short that all columns fit are indexed by the column itself.
+ * waves != 0 asks for the shape of that many wavefronts per block (the
+ * autotuner's candidates; fewer rows than CUs then do not rule it out). */
 static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long long est,
-                       int known, int grows, bmlh_spgemm_shape *out)
+                       int known, int grows, int waves, bmlh_spgemm_shape *out)
 {
     if (N <= 0 || span <= 0)
         return 0;
@@ -82,7 +84,7 @@ static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long lo
     long long best_lds = 0;
     for (int w = 8; w >= 1; w--) {
         const int rb = w * (64 / g);
-        if (w > 1 && (long long) N < 256ll * rb)
+        if (waves ? w != waves : w > 1 && (long long) N < 256ll * rb)
             continue; /* fewer blocks than CUs */
         long long D = est + est * 15 * (rb - 1) / 100 + 32;
         if (dense || D > span)
@@ -133,8 +135,10 @@ static int shape_from_env(void)
     return 0;
 }
 
-void bmlh_pick_spgemm(int precision, int N, int span, int max_a, int max_b, int touched_hint,
-                      int hint_max_a, int flags, bmlh_spgemm_shape *out)
+/* bmlh_pick_spgemm; direct_waves != 0: where it takes the direct kernel, its
+ * shape of that many wavefronts per block */
+static void pick(int precision, int N, int span, int max_a, int max_b, int touched_hint,
+                 int hint_max_a, int flags, int direct_waves, bmlh_spgemm_shape *out)
 {
     const int square = flags & BMLH_PICK_SQUARE;
     int g = 8;
@@ -312,7 +316,13 @@ void bmlh_pick_spgemm(int precision, int N, int span, int max_a, int max_b, int 
      * LDS holds a row (a shape from the environment is the hash kernels') */
     if (engine == BMLHIP_ROW_EXACT && !shape_from_env())
         pick_direct(bmlh_elem_size(precision), N, span, max_a, max_b, est, touched_hint > 0,
-                    touched_hint > 0 && 20 * max_a > 21 * hint_max_a, out);
+                    touched_hint > 0 && 20 * max_a > 21 * hint_max_a, direct_waves, out);
+}
+
+void bmlh_pick_spgemm(int precision, int N, int span, int max_a, int max_b, int touched_hint,
+                      int hint_max_a, int flags, bmlh_spgemm_shape *out)
+{
+    pick(precision, N, span, max_a, max_b, touched_hint, hint_max_a, flags, 0, out);
 }
 
 /* ---- measured shapes ------------------------------------------------------
@@ -530,17 +540,16 @@ void bmlh_tuned_spgemm(int precision, int N, int max_a, int max_b, int touched_h
                 try_shape(&c, &best, &best_ms, fn, ctx);
         }
     } else if (out->engine == BMLHIP_ROW_DIRECT) {
-        /* wavefronts per block and the LDS that goes with them */
-        const int w0 = best.waves, t0 = best.table;
+        /* wavefronts per block, each with the LDS that its rows need (the
+         * index at its head does not shrink with them); counts whose LDS
+         * cannot hold a row are no candidates */
+        const int w0 = best.waves;
         for (int w = w0 > 1 ? w0 / 2 : 1; w <= 2 * w0 && w <= 8; w *= 2) {
             if (w == w0)
                 continue;
-            c = best;
-            c.waves = w;
-            c.table = (int) ((long long) t0 * w / w0);
-            if (c.table > 160 * 1024)
-                c.table = 160 * 1024;
-            try_shape(&c, &best, &best_ms, fn, ctx);
+            pick(precision, N, N, max_a, max_b, touched_hint, hint_max_a, flags, w, &c);
+            if (c.engine == BMLHIP_ROW_DIRECT && c.waves == w)
+                try_shape(&c, &best, &best_ms, fn, ctx);
         }
     } else {
         static const int bk[] = {2, 4, 8};

@@ -77,3 +77,34 @@ def test_search_from_one_wavefront_ends():
     here = os.path.dirname(os.path.abspath(__file__))
     env = dict(os.environ, PYTHONPATH=os.pathsep.join([here, os.path.dirname(here)]))
     subprocess.run([sys.executable, "-c", code], check=True, timeout=60, env=env)
+
+
+def rows_held(prec, sh, D):
+    """Rows of D columns that the kernel's LDS holds at once: the index words
+    and 48 bytes, the columns' list (2^16 columns or more), a spare slot per
+    lane, and per row its sums and its 16-bit list."""
+    def up(b):
+        return (b + 15) // 16 * 16
+    head = up(8 * (sh.wrows // 32 + 2)) + 48
+    fixed = (up(4 * D) if sh.wrows > 65536 else 0) + 64 * sh.waves * ELEM[prec]
+    per_row = up(D * ELEM[prec]) + up(2 * D)
+    return max(0, sh.table - head - fixed) // per_row
+
+
+DENSE = 1  # numbering: a column is its own slot
+
+
+@pytest.mark.parametrize("prec", sorted(ELEM))
+def test_every_candidate_holds_a_row(tuner, prec):
+    """A shape whose LDS holds no row hands every row to the global-table
+    pass; it must not be measured, however fast that is."""
+    for N in list(range(60, 3000, 97)) + [870, 946, 1000, 1072, 1716, 2817, 2892, 4096, 30000]:
+        for n, touched in ((9, 0), (9, 60), (33, 0), (33, 300), (63, 0), (63, min(N, 1500))):
+            hip.autotune_clear()
+            sh, tried = search(prec, N, n, touched, ms=lambda s: float(s.waves))
+            for c in tried:
+                if c.engine != DIRECT:
+                    continue
+                D = N if c.wbits == DENSE else min(touched or 1, N)
+                assert rows_held(prec, c, D) >= 1, (N, n, touched, c.key())
+                assert c.table <= 160 * 1024 and c.wrows == N

@@ -101,3 +101,18 @@ def test_autotuned_sp2_window_engine(hip, tmp_path):
     assert r1.iterations == r0.iterations
     np.testing.assert_array_equal(h1[:, 3], h0[:, 3])
     assert np.abs(X1.get().to_dense() - X0.get().to_dense()).max() <= 1e-9
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64, np.complex128])
+@pytest.mark.parametrize("N", [100, 500, 1000, 2817, 4096])
+def test_autotuned_direct_kernel_forms_every_row(tuned, N, dtype):
+    """Whatever shape of the direct kernel the search takes, from shapes of
+    one wavefront to rows that index every column, the product is whole."""
+    hip, _ = tuned
+    A = G.random_ell(N, 40, min(33, N // 2), 7, dtype)
+    M = min(N, 1300)
+    ref, _ = orc.x2(A, M, 1e-3)
+    for k in range(2):  # searched, then from the table
+        X2 = hip.zero_matrix(A.precision, N, M)
+        hip.multiply_x2(hip.from_ell(A), X2, 1e-3)
+        assert_ell_identical(X2.get(), ref, f"tuned x2 N={N} run {k}")
