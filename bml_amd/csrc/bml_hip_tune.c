@@ -498,7 +498,17 @@ void bmlh_tuned_spgemm(int precision, int N, int max_a, int max_b, int touched_h
              qbucket(touched_hint));
     for (int k = 0; k < g_ntab; k++)
         if (!strcmp(g_tab[k].key, key)) {
-            *out = g_tab[k].sh;
+            /* a key stands for sizes up to a fifth apart.  The direct
+             * kernel's index and LDS are made for one: its entries give the
+             * wavefronts, the rest follows from this call's own sizes (and
+             * where that many do not fit, the analytic shape stays) */
+            bmlh_spgemm_shape c = g_tab[k].sh;
+            if (c.engine == BMLHIP_ROW_DIRECT) {
+                pick(precision, N, N, max_a, max_b, touched_hint, hint_max_a, flags, c.waves, &c);
+                if (c.engine != BMLHIP_ROW_DIRECT || c.waves != g_tab[k].sh.waves)
+                    return;
+            }
+            *out = c;
             return;
         }
     bmlh_spgemm_shape best = *out;

@@ -108,3 +108,41 @@ def test_every_candidate_holds_a_row(tuner, prec):
                 D = N if c.wbits == DENSE else min(touched or 1, N)
                 assert rows_held(prec, c, D) >= 1, (N, n, touched, c.key())
                 assert c.table <= 160 * 1024 and c.wrows == N
+
+
+@pytest.mark.parametrize("prec,N,N2,n", [(SINGLE, 1300, 1400, 33), (DOUBLE, 900, 1000, 33),
+                                         (DOUBLE, 870, 1020, 40), (SINGLE, 1500, 1700, 33),
+                                         (DOUBLE_C, 900, 1000, 33), (DOUBLE, 20000, 22000, 33)])
+def test_cached_shape_fits_the_call(tuner, prec, N, N2, n):
+    """An entry of the table serves sizes near its own; the shape taken from
+    it is the call's own size's, in both orders."""
+    for first, second in ((N, N2), (N2, N)):
+        hip.autotune_clear()
+        assert search(prec, first, n, ms=lambda s: float(s.waves))[1]
+        sh, tried = search(prec, second, n)
+        assert not tried, "not the same key"
+        assert sh.engine == DIRECT and sh.wrows == second
+        D = second if sh.wbits == DENSE else min(1000, second)
+        assert rows_held(prec, sh, D) >= 1
+
+
+def test_direct_entry_of_a_file_is_not_taken_as_it_stands(tmp_path):
+    """Wavefronts that do not fit, an index for other columns or an LDS size
+    from a cache file never reach the kernel."""
+    p = tmp_path / "tune.txt"
+    hip.autotune_clear()
+    hip.set_autotune(True, str(p))
+    try:
+        search(DOUBLE, 1000, 33)
+        key = p.read_text().split()[0]
+        for waves in (0, 1, 2, 7, 9, 4096, -3):
+            p.write_text(f"{key} 64 2048 1 0 {waves} 3 1 17 0.001\n")
+            hip.autotune_clear()
+            hip.set_autotune(True, str(p))
+            sh, tried = search(DOUBLE, 1000, 33)
+            assert not tried
+            assert sh.engine == DIRECT and sh.wrows == 1000 and 1 <= sh.waves <= 8
+            assert rows_held(DOUBLE, sh, 1000) >= 1
+    finally:
+        hip.set_autotune(False, "")
+        hip.autotune_clear()

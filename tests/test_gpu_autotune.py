@@ -116,3 +116,20 @@ def test_autotuned_direct_kernel_forms_every_row(tuned, N, dtype):
         X2 = hip.zero_matrix(A.precision, N, M)
         hip.multiply_x2(hip.from_ell(A), X2, 1e-3)
         assert_ell_identical(X2.get(), ref, f"tuned x2 N={N} run {k}")
+
+
+@pytest.mark.parametrize("dtype,N,N2", [(np.float32, 1300, 1400), (np.float64, 900, 1000),
+                                        (np.float64, 870, 1020), (np.float32, 1500, 1700)])
+def test_tuned_shape_serves_another_size(tuned, dtype, N, N2):
+    """Two sizes of one key, in both orders: the second product takes the
+    first one's entry and is whole."""
+    hip, _ = tuned
+    for sizes in ((N, N2), (N2, N)):
+        hip.autotune_clear()
+        for n in sizes:
+            A = G.random_ell(n, 40, 33, n, dtype)
+            ref, _ = orc.x2(A, n, 1e-3)
+            X2 = hip.zero_matrix(A.precision, n, n)
+            hip.multiply_x2(hip.from_ell(A), X2, 1e-3)
+            assert_ell_identical(X2.get(), ref, f"N={n} of {sizes}")
+        assert hip.autotune_entries() == 1
