@@ -3514,8 +3514,9 @@ int spgemm_typed(const bmlhip_spgemm_args *a) {
         p.qinfo = a->batch->d_qinfo;
     }
     int *fill = nullptr;
+    bool whole = false;
     if (direct) {
-        rc = launch_rowdir<T>(p, a->group, a->bucket, a->waves, a->table, a->wrows, a->wbits, s);
+        rc = launch_rowdir<T>(p, a->group, a->bucket, a->waves, a->table, a->wrows, a->wbits, s, &whole);
     } else if (sym) {
         fill = (int *) bmlhip_scratch_zeroed(BMLHIP_SYMFILL_SLOT, sizeof(int) * (size_t) (a->N + 1));
         if (!fill) return fail_msg(4, "scratch allocation failed");
@@ -3551,9 +3552,7 @@ int spgemm_typed(const bmlhip_spgemm_args *a) {
         return fail_msg(2, "group %d not one of 8/16/32/64", a->group);
     }
     if (rc) return rc;
-    // (the direct kernel on columns that are their own slots has room for
-    // every row: see pick_direct)
-    if (!(direct && a->wbits == BMLHIP_DIR_DENSE)) {
+    if (!whole) {
         hipLaunchKernelGGL(k_spgemm_global<T>, dim3(gblocks), dim3(64), 0, s, p, (unsigned) gsize,
                            gtab, cursor);
         if ((rc = report("k_spgemm_global"))) return rc;

@@ -91,7 +91,7 @@ __device__ __forceinline__ bool is_taken(const cf64 *s) { return (*(const word2 
 
 __device__ __forceinline__ uint64_t ballotb(bool b) { return __builtin_amdgcn_ballot_w64(b); }
 
-__device__ __forceinline__ unsigned up16(unsigned b) { return (b + 15u) & ~15u; }
+__host__ __device__ __forceinline__ unsigned up16(unsigned b) { return (b + 15u) & ~15u; }
 
 __device__ __forceinline__ unsigned slot_of(const uint2 *idx0, unsigned col) {
     const uint2 e = idx0[col >> 5];
@@ -709,7 +709,7 @@ namespace bmlhip {
 
 template <typename T>
 int launch_rowdir(const SpParams &p, int group, int nch, int waves, int lds, int span, int mode,
-                  hipStream_t s) {
+                  hipStream_t s, bool *whole) {
     // what the kernel assumes of its LDS: the index words and, in the rest,
     // the bitmap of A's columns and at least a short list
     const long long words = span / 32 + 2;
@@ -718,6 +718,14 @@ int launch_rowdir(const SpParams &p, int group, int nch, int waves, int lds, int
         bmlhip_set_errmsg("direct row product: launch shape out of range");
         return 2;
     }
+    // Every row is formed here when a row of all reachable columns fits (the
+    // kernel's layout; a batch's range starts at a multiple of 32 columns) and
+    // all are numbered: how many are touched depends on the data.
+    const unsigned D = (unsigned) (p.row_sys ? span + 31 : p.N);
+    const unsigned need = up16(8u * (unsigned) words) + 48u + 64u * (unsigned) waves * (unsigned) sizeof(T) +
+                          up16(D * (unsigned) sizeof(T)) + up16(2u * D);
+    *whole = mode == BMLHIP_DIR_DENSE && D <= 65535u && (D + 31u) / 32u <= (unsigned) words &&
+             need <= (unsigned) lds;
     switch (group * 8 + nch) {
     case 8 * 8 + 1: return launch<T, 8, 1>(p, waves, lds, span, mode, s);
     case 16 * 8 + 1: return launch<T, 16, 1>(p, waves, lds, span, mode, s);
@@ -733,9 +741,9 @@ int launch_rowdir(const SpParams &p, int group, int nch, int waves, int lds, int
     return 2;
 }
 
-template int launch_rowdir<float>(const SpParams &, int, int, int, int, int, int, hipStream_t);
-template int launch_rowdir<double>(const SpParams &, int, int, int, int, int, int, hipStream_t);
-template int launch_rowdir<cf32>(const SpParams &, int, int, int, int, int, int, hipStream_t);
-template int launch_rowdir<cf64>(const SpParams &, int, int, int, int, int, int, hipStream_t);
+template int launch_rowdir<float>(const SpParams &, int, int, int, int, int, int, hipStream_t, bool *);
+template int launch_rowdir<double>(const SpParams &, int, int, int, int, int, int, hipStream_t, bool *);
+template int launch_rowdir<cf32>(const SpParams &, int, int, int, int, int, int, hipStream_t, bool *);
+template int launch_rowdir<cf64>(const SpParams &, int, int, int, int, int, int, hipStream_t, bool *);
 
 }  // namespace bmlhip

@@ -81,9 +81,10 @@ __device__ __forceinline__ T bcast(T v, int src) {
 // (8, 16, 32 or 64), nch chunks of a row of B per step, waves wavefronts per
 // block, lds bytes of LDS per block, span = columns a block's rows can reach
 // (N, or for batched systems the columns of the systems a block can touch),
-// mode: BMLHIP_DIR_*.
+// mode: BMLHIP_DIR_*.  *whole: this shape leaves no row to the global-table
+// pass.
 template <typename T>
 int launch_rowdir(const SpParams &p, int group, int nch, int waves, int lds, int span, int mode,
-                  hipStream_t s);
+                  hipStream_t s, bool *whole);
 
 }  // namespace bmlhip
