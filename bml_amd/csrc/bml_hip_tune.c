@@ -313,8 +313,9 @@ static void pick(int precision, int N, int span, int max_a, int max_b, int touch
      * ran 1.3x slower than the hardware's round-robin order */
     out->remap = (e = getenv("BML_HIP_XCD_REMAP")) ? atoi(e) : 0;
     /* the exact engine's work goes to the direct-index kernel wherever its
-     * LDS holds a row (a shape from the environment is the hash kernels') */
-    if (engine == BMLHIP_ROW_EXACT && !shape_from_env())
+     * LDS holds a row (a shape from the environment is the hash kernels', and
+     * so is a batch's work queue) */
+    if (engine == BMLHIP_ROW_EXACT && !(flags & BMLH_PICK_QUEUE) && !shape_from_env())
         pick_direct(bmlh_elem_size(precision), N, span, max_a, max_b, est, touched_hint > 0,
                     touched_hint > 0 && 20 * max_a > 21 * hint_max_a, direct_waves, out);
 }

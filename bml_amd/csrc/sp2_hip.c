@@ -634,7 +634,7 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
         const int mx = cur->aux->stats_valid ? cur->aux->max_nnz : cur->M;
         bmlh_spgemm_shape sh;
         bmlh_pick_spgemm(cur->matrix_precision, N, span, mx, mx, touched, hint_max,
-                         BMLH_PICK_SQUARE, &sh);
+                         BMLH_PICK_SQUARE | (d.b.d_list ? BMLH_PICK_QUEUE : 0), &sh);
         if (o.graph) {
             /* replay the iteration as a graph; capture anew when the launch
              * shape or the precision changes (the first pass runs eagerly so

@@ -146,3 +146,16 @@ def test_direct_entry_of_a_file_is_not_taken_as_it_stands(tmp_path):
     finally:
         hip.set_autotune(False, "")
         hip.autotune_clear()
+
+
+@pytest.mark.parametrize("prec", sorted(ELEM))
+def test_a_work_queue_gets_the_hash_kernels(prec):
+    """Rows taken from a batch's work queue (BML_HIP_BATCH_QUEUE=1): the
+    direct kernel, whose blocks form consecutive rows, does not read it."""
+    queue = 4
+    for N, span, n, touched in ((3000, 900, 7, 0), (38394, 8190, 63, 500), (512, 64, 9, 30)):
+        sh, out = Shape(), Shape()
+        hip.lib().bmlh_pick_spgemm(prec, N, span, n, n, touched, n, SQUARE, C.byref(sh))
+        assert sh.engine == DIRECT
+        hip.lib().bmlh_pick_spgemm(prec, N, span, n, n, touched, n, SQUARE | queue, C.byref(out))
+        assert out.engine == EXACT and out.group in (8, 16, 32, 64) and out.table >= 64
