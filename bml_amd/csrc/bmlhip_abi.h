@@ -132,7 +132,8 @@ bmlhip_host *bmlhip_host_dev(void);
 /* the last queued operation wrote its status to the host and left the status
  * block clear */
 void bmlhip_status_published(void);
-/* the status block is clear for an operation that ends with k_tail */
+/* the status block is clear for an operation that begins now and ends with
+ * k_tail; until that is queued the block counts as in use */
 int bmlhip_status_ready(void);
 /* wait, then the state of the last BMLHIP_TAIL_CHECK / _CHECK_BATCH */
 int bmlhip_sp2_state_fetch(bmlhip_sp2_state *st);

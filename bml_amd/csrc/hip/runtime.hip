@@ -352,10 +352,11 @@ bmlhip_host *bmlhip_host_dev(void) { return g.host; }
 void bmlhip_status_published(void) { g.clear = g.published = true; }
 
 int bmlhip_status_ready(void) {
-    if (g.clear) return 0;
-    const int rc = bmlhip_status_reset();
-    g.clear = rc == 0;
-    return rc;
+    if (!g.clear) return bmlhip_status_reset();
+    // the operation that begins here fills the block: only its own k_tail
+    // says that it is clear again and that host->status is current
+    g.clear = g.published = false;
+    return 0;
 }
 
 int bmlhip_status_reset(void) {
