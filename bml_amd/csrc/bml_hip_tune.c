@@ -33,6 +33,51 @@
 #include <stdlib.h>
 #include <string.h>
 
+/* Where the direct-index kernel is the faster one.  Every block of it pays
+ * for an index of all reachable columns (8 bytes of LDS and a share of a scan
+ * per 32 of them), and rows that share a block hold a sum for each column
+ * that any of them touches; the hash kernels pay per product.  Measured with
+ * both kernels on random rows near the diagonal and all over the matrix, on
+ * lattice Hamiltonians and iterates, in three element types (us, double
+ * unless said, hash and direct):
+ *
+ * - up to 2^14 columns the index is small: direct, 2 to 4 times as fast from
+ *   9 entries a row on (N = 16384: 31 near the diagonal 444 and 121, all
+ *   over 590 and 323), level on shorter ones;
+ * - rows of more than 64 entries: direct (N = 25000, 100 near the diagonal
+ *   9878 and 2540; 64^3 lattice, 185 a row 48500 and 31100).  Above 2^17
+ *   columns the index leaves few rows per CU: with the counts of an earlier
+ *   product known, so that the hash table has its right size, it wins below
+ *   span / 32 products a row (64^3, 87 a row: 8920 and 9400) and where less
+ *   than two and a half rows fit beside the index (complex, 322 a row, 64^3:
+ *   179 ms and 243, 56^3: 181 and 84);
+ * - 33 to 64 entries: direct up to 2^16 columns (N = 65000, 45 near the
+ *   diagonal 1560 and 850, all over 10000 and 6950), above that on rows known
+ *   to share columns, up to 2^17 (N = 262144, 45: 6160 and 6290; not known,
+ *   complex, N = 100000, 64: 7530 and 11430), and where the row does not fit
+ *   the hash kernel's table (all over, N = 262144, 45: 42400 and 32800);
+ * - up to 32 entries, several rows to a wavefront: only on rows known to
+ *   share columns (fewer distinct ones than 7/10 of the products), up to
+ *   2^17 columns and 350 for each product of a row (48^3 lattice: 25 a row
+ *   875 and 690, 7 a row 151 and 333; all over, N = 32000, 12: 148 and 269). */
+static int direct_wins(size_t es, int span, int max_a, int max_b, long long est, int known)
+{
+    const long long products = (long long) max_a * max_b;
+    if (span <= 16384)
+        return 1;
+    const int shared = known && 10 * est <= 7 * products;
+    if (max_b > 64)
+        return !known || span <= 131072 ||
+               (32 * products >= span &&
+                5 * est * (long long) (es + 2) <= 2 * (160 * 1024 - span / 4));
+    if (max_b > 32) {
+        if (span <= 65536 || (known && est * 5 / 4 * (long long) (es + 6) > 32 * 1024))
+            return 1;
+        return shared && span <= 131072;
+    }
+    return shared && span <= 131072 && 350 * products >= span;
+}
+
 /* Shape of the direct-index kernel (hip/rowdir.hip), 0 when its LDS cannot
  * hold one row.
  *
@@ -42,18 +87,19 @@
  * step.  W wavefronts per block and the blocks per CU follow the LDS: the
  * block needs 8 bytes per 32 reachable columns, and each row sizeof(T) + 2 per
  * column that any row of the block touches (15% more for each further row: on
- * a lattice a step along the fast axis adds the ball's cross-section); the W with the most wavefronts per CU is taken, the larger
- * of equals (its rows share more of the index).  A block whose rows touch
- * more than that forms them in several passes, so a wrong guess costs time
- * only; without a hint the bound min(span, max_a * max_b) is far above the
- * truth, and 3000 columns are the most that are provided for.
+ * a lattice a step along the fast axis adds the ball's cross-section); the W
+ * with the most wavefronts per CU is taken, the larger of equals (its rows
+ * share more of the index).  A block whose rows touch more than that forms
+ * them in several passes, so a wrong guess costs time only; without a hint
+ * the bound min(span, max_a * max_b) is far above the truth, and 3000 columns
+ * are the most that are provided for.
  * Rows so short that all columns fit are indexed by the column itself.
  * waves != 0 asks for the shape of that many wavefronts per block (the
  * autotuner's candidates; fewer rows than CUs then do not rule it out). */
 static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long long est,
                        int known, int grows, int waves, bmlh_spgemm_shape *out)
 {
-    if (N <= 0 || span <= 0)
+    if (N <= 0 || span <= 0 || !direct_wins(es, span, max_a, max_b, est, known))
         return 0;
     int g = 8;
     while (g < 64 && (g < max_b || (long long) N * g < 64 * 2048))

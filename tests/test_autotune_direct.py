@@ -159,3 +159,27 @@ def test_a_work_queue_gets_the_hash_kernels(prec):
         assert sh.engine == DIRECT
         hip.lib().bmlh_pick_spgemm(prec, N, span, n, n, touched, n, SQUARE | queue, C.byref(out))
         assert out.engine == EXACT and out.group in (8, 16, 32, 64) and out.table >= 64
+
+
+# (precision, N, entries a row, distinct columns a row of an earlier product
+# or 0, direct kernel): the sides of each line of the rule
+CROSSOVER = [
+    (DOUBLE, 16384, 7, 0, True), (DOUBLE, 16385, 7, 0, False), (DOUBLE, 16385, 32, 0, False),
+    (DOUBLE, 17150, 7, 25, True), (DOUBLE, 17151, 7, 25, False), (DOUBLE, 17151, 7, 43, False),
+    (DOUBLE, 110592, 25, 87, True), (DOUBLE, 262144, 25, 87, False), (DOUBLE, 262144, 7, 25, False),
+    (DOUBLE, 32000, 12, 133, False), (DOUBLE, 32000, 12, 99, True),
+    (DOUBLE, 65536, 33, 0, True), (DOUBLE, 65537, 33, 0, False), (DOUBLE, 65537, 64, 0, False),
+    (DOUBLE, 131072, 45, 639, True), (DOUBLE, 131073, 45, 639, False),
+    (DOUBLE, 262144, 45, 1981, True), (SINGLE, 262144, 45, 1981, False),
+    (DOUBLE_C, 100000, 64, 0, False), (DOUBLE_C, 100000, 64, 949, True),
+    (DOUBLE, 70001, 65, 0, True), (DOUBLE, 262144, 87, 260, False), (DOUBLE, 262144, 87, 0, True),
+    (DOUBLE, 262144, 185, 1177, True), (DOUBLE_C, 262144, 322, 2300, False),
+    (DOUBLE_C, 175616, 322, 2300, True), (SINGLE_C, 262144, 322, 2300, True),
+]
+
+
+@pytest.mark.parametrize("prec,N,n,touched,direct", CROSSOVER)
+def test_crossover_of_the_two_exact_kernels(prec, N, n, touched, direct):
+    """Large matrices of short rows, and short rows all over the matrix, stay
+    on the hash kernels."""
+    assert (analytic(prec, N, n, touched).engine == DIRECT) == direct

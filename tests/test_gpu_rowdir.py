@@ -131,3 +131,13 @@ def test_overflow_is_reported(hip):
     X2 = hip.zero_matrix(A.precision, 40, 39)
     with pytest.raises(hip.BmlError, match="Number of non-zeroes per row > M"):
         hip.multiply_x2(hip.from_ell(A), X2, 0.0)
+
+
+@pytest.mark.parametrize("N", [65535, 65536, 65537, 70001])
+@pytest.mark.parametrize("dtype", [np.float64, np.complex64])
+def test_many_columns_long_rows(hip, dtype, N):
+    """Above 2^16 columns the list holds slots instead of columns: rows long
+    enough for the direct kernel there."""
+    A = G.random_banded(N=N, M=90, draws=36, band=60, seed=3, dtype=dtype)
+    assert A.nnz.max() > 64
+    square(hip, A, 260, 1e-3)
