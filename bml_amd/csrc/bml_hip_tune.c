@@ -87,12 +87,16 @@ static int direct_wins(size_t es, int span, int max_a, int max_b, long long est,
  * step.  W wavefronts per block and the blocks per CU follow the LDS: the
  * block needs 8 bytes per 32 reachable columns, and each row sizeof(T) + 2 per
  * column that any row of the block touches (15% more for each further row: on
- * a lattice a step along the fast axis adds the ball's cross-section); the W
- * with the most wavefronts per CU is taken, the larger of equals (its rows
- * share more of the index).  A block whose rows touch more than that forms
- * them in several passes, so a wrong guess costs time only; without a hint
- * the bound min(span, max_a * max_b) is far above the truth, and 3000 columns
- * are the most that are provided for.
+ * a lattice a step along the fast axis adds the ball's cross-section; as many
+ * again where up to 16 entries share a wavefront with other rows and are not
+ * known to share columns with them); the W with the most wavefronts per CU is
+ * taken, the larger of equals (its rows share more of the index).  A block
+ * whose rows touch more than that forms them in several passes; a row that
+ * does not fit alone is left to the global-table pass.  Without a hint the
+ * bound min(span, max_a * max_b) is mostly far above the truth: 3000 columns
+ * are provided for, 6500 for rows of more than 64 entries, whose hash tables
+ * held as many (double, N = 16384, 80 entries all over: 20.8 ms with 3000,
+ * 4.2 with 6500, the hash kernel 8.7; near the diagonal 0.99, 1.75, 5.3).
  * Rows so short that all columns fit are indexed by the column itself.
  * waves != 0 asks for the shape of that many wavefronts per block (the
  * autotuner's candidates; fewer rows than CUs then do not rule it out). */
@@ -118,21 +122,33 @@ static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long lo
         est = span;
     const long long per = (long long) es + 2;
     const int dense = span * per <= 6 * 1024 || (2 * est >= span && span * per <= 20 * 1024);
-    if (!known && est > 3000)
-        est = 3000;
+    const int shared = known && 10 * est <= 7 * (long long) max_a * max_b;
+    const long long words = span / 32 + 2;
+    const long long cu = 160 * 1024;
+    if (!known) {
+        /* at most what the LDS holds beside the index */
+        const long long room = (cu - 8 * words - 64 * (long long) es - 192) /
+                                   (per + (span > 65536 ? 4 : 0)) - 40;
+        long long most = max_b > 64 ? 6500 : 3000;
+        if (most > room)
+            most = room;
+        if (most < 3000)
+            most = 3000;
+        if (est > most)
+            est = most;
+    }
     /* growing rows touch more columns for their length each time (a ball of
      * radius r squared has radius 2r) */
     if (grows && est + est / 2 <= span)
         est += est / 2;
-    const long long words = span / 32 + 2;
-    const long long cu = 160 * 1024;
+    const int more = g <= 16 && !shared ? 100 : 15;
     int best = 0, best_waves = 0;
     long long best_lds = 0;
     for (int w = 8; w >= 1; w--) {
         const int rb = w * (64 / g);
         if (waves ? w != waves : w > 1 && (long long) N < 256ll * rb)
             continue; /* fewer blocks than CUs */
-        long long D = est + est * 15 * (rb - 1) / 100 + 32;
+        long long D = est + est * more * (rb - 1) / 100 + 32;
         if (dense || D > span)
             D = span;
         long long need = 8 * words + 64 + (span > 65536 ? 4 * D + 16 : 0) + 64ll * w * (long long) es +

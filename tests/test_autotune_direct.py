@@ -183,3 +183,22 @@ def test_crossover_of_the_two_exact_kernels(prec, N, n, touched, direct):
     """Large matrices of short rows, and short rows all over the matrix, stay
     on the hash kernels."""
     assert (analytic(prec, N, n, touched).engine == DIRECT) == direct
+
+
+@pytest.mark.parametrize("prec", sorted(ELEM))
+def test_lds_for_rows_not_known_to_share_columns(prec):
+    """Rows of more than 64 entries whose product is not known: LDS for 6500
+    columns (or all that they can touch), or as many as fit beside the
+    index.  Short rows: for the columns of every row of the block."""
+    for N, n in ((3500, 100), (8000, 100), (16384, 80), (25000, 140), (100000, 90)):
+        sh = analytic(prec, N, n)
+        room = (160 * 1024 - 8 * (N // 32 + 2)) // (ELEM[prec] + 2) - 200
+        if N > 65536:
+            room = room * 2 // 3
+        assert sh.engine == DIRECT
+        assert rows_held(prec, sh, min(N, n * n, 6500, room)) >= 1, (N, n, sh.key())
+    for N, n, touched in ((12000, 7, 0), (16384, 12, 133), (16384, 16, 241), (9000, 9, 75)):
+        sh = analytic(prec, N, n, touched)
+        rb = sh.waves * (64 // sh.group)
+        assert sh.engine == DIRECT and sh.group <= 16
+        assert rows_held(prec, sh, rb * (touched or n * n)) >= rb, (N, n, sh.key())
