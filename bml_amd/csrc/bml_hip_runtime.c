@@ -222,6 +222,11 @@ void bml_hip_synchronize(void)
     check_status("bml_hip_synchronize", &st);
 }
 
+void bml_hip_release_temporaries(void)
+{
+    bmlhip_temp_release();
+}
+
 void *bml_hip_stream(void)
 {
     if (bmlh_ready())

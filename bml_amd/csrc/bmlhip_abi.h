@@ -72,6 +72,8 @@ void bmlhip_free(void *d_ptr);
  * order (bounded; either free takes either kind) */
 int bmlhip_temp_malloc(void **d_ptr, size_t bytes);
 void bmlhip_temp_free(void *d_ptr);
+/* the kept blocks back to the device */
+void bmlhip_temp_release(void);
 int bmlhip_h2d(void *d_dst, const void *src, size_t bytes);
 int bmlhip_d2h(void *dst, const void *d_src, size_t bytes);
 int bmlhip_d2d(void *d_dst, const void *d_src, size_t bytes);

@@ -38,8 +38,8 @@ Runtime g;
 // that a free needs took 0.6 - 5 ms of a 3001-block-row bml_multiply whose
 // kernels run 0.2 ms.  Freed blocks are kept, up to POOL_BLOCKS of them and
 // POOL_BYTES in all, and handed out again in stream order (all work runs on
-// one stream).  They go back to the device when an allocation fails and at
-// shutdown.
+// one stream).  They go back to the device when an allocation fails, at
+// bml_hip_release_temporaries and at shutdown.
 constexpr size_t POOL_BYTES = (size_t) 16 << 30;
 constexpr size_t POOL_BLOCKS = 64;
 struct PoolBlock {
@@ -267,6 +267,11 @@ void bmlhip_temp_free(void *p) {
         }
     }
     bmlhip_free(p);
+}
+
+void bmlhip_temp_release(void) {
+    std::lock_guard<std::mutex> hold(pool_lock);
+    pool_release();
 }
 
 void bmlhip_free(void *p) {

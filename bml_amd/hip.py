@@ -88,6 +88,7 @@ _SIGS = {
     "bml_hip_last_error": (_I, [C.c_char_p, _I]),
     "bml_hip_clear_error": (None, []),
     "bml_hip_synchronize": (None, []),
+    "bml_hip_release_temporaries": (None, []),
     "bml_hip_stream": (_P, []),
     "bml_hip_version": (C.c_char_p, []),
     "bml_hip_set_autotune": (None, [_I, C.c_char_p]),
@@ -226,6 +227,11 @@ def init(device: int = 0) -> None:
 
 def synchronize() -> None:
     _call("bml_hip_synchronize")
+
+
+def release_temporaries() -> None:
+    """Give the device memory kept for the temporaries of later calls back."""
+    _call("bml_hip_release_temporaries")
 
 
 def stream() -> int:

@@ -124,6 +124,12 @@ int bml_hip_last_error(char *buf, int len);
 void bml_hip_clear_error(void);
 /* Wait for all queued work and run the deferred overflow checks. */
 void bml_hip_synchronize(void);
+/* Give the device memory of finished temporaries back.  Calls that need a
+ * matrix of their own (bml_multiply into its operand, the SP2 drivers, the
+ * block multiply) keep its arrays for the next such call: at most 64 blocks
+ * and 16 GiB, which other allocators of the process cannot use meanwhile.
+ * Waits for the queued work.  No bml counterpart. */
+void bml_hip_release_temporaries(void);
 /* The hipStream_t every kernel of the library runs on. */
 void *bml_hip_stream(void);
 /* Library build string. */
