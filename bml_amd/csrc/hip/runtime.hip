@@ -7,7 +7,6 @@
 
 #include <mutex>
 #include <unordered_map>
-#include <vector>
 
 #include "../bmlhip_abi.h"
 
@@ -47,17 +46,28 @@ struct PoolBlock {
     size_t n;
 };
 std::mutex pool_lock;
-std::vector<PoolBlock> pool_kept;
-size_t pool_kept_bytes = 0;
+PoolBlock pool_kept[POOL_BLOCKS];
+size_t pool_nkept = 0, pool_kept_bytes = 0;
 std::unordered_map<void *, size_t> pool_live;
 
 // (pool_lock held)
 void pool_release() {
-    if (pool_kept.empty()) return;
+    if (!pool_nkept) return;
     (void) hipStreamSynchronize(g.stream);
-    for (const PoolBlock &b : pool_kept) (void) hipFree(b.p);
-    pool_kept.clear();
-    pool_kept_bytes = 0;
+    for (size_t k = 0; k < pool_nkept; k++) (void) hipFree(pool_kept[k].p);
+    pool_nkept = pool_kept_bytes = 0;
+}
+
+// Notes a block in use (pool_lock held); false when the host has no memory
+// for the note: such a block is freed as any other array.  The callers are C,
+// which no exception may reach.
+bool pool_note(void *p, size_t n) noexcept {
+    try {
+        pool_live[p] = n;
+        return true;
+    } catch (...) {
+        return false;
+    }
 }
 
 // hipMalloc; when it fails, once more with the pool given back
@@ -232,24 +242,22 @@ int bmlhip_temp_malloc(void **p, size_t bytes) {
     {
         // the smallest kept block that is not much too large
         std::lock_guard<std::mutex> hold(pool_lock);
-        size_t best = pool_kept.size();
-        for (size_t k = 0; k < pool_kept.size(); k++)
+        size_t best = pool_nkept;
+        for (size_t k = 0; k < pool_nkept; k++)
             if (pool_kept[k].n >= bytes && pool_kept[k].n <= 2 * bytes + 65536 &&
-                (best == pool_kept.size() || pool_kept[k].n < pool_kept[best].n))
+                (best == pool_nkept || pool_kept[k].n < pool_kept[best].n))
                 best = k;
-        if (best < pool_kept.size()) {
+        if (best < pool_nkept && pool_note(pool_kept[best].p, pool_kept[best].n)) {
             *p = pool_kept[best].p;
-            pool_live[*p] = pool_kept[best].n;
             pool_kept_bytes -= pool_kept[best].n;
-            pool_kept[best] = pool_kept.back();
-            pool_kept.pop_back();
+            pool_kept[best] = pool_kept[--pool_nkept];
             return 0;
         }
     }
     const int rc = bmlhip_malloc(p, bytes);
     if (rc) return rc;
     std::lock_guard<std::mutex> hold(pool_lock);
-    pool_live[*p] = bytes;
+    (void) pool_note(*p, bytes);
     return 0;
 }
 
@@ -258,9 +266,9 @@ void bmlhip_temp_free(void *p) {
     {
         std::lock_guard<std::mutex> hold(pool_lock);
         const auto it = pool_live.find(p);
-        if (it != pool_live.end() && pool_kept.size() < POOL_BLOCKS &&
+        if (it != pool_live.end() && pool_nkept < POOL_BLOCKS &&
             pool_kept_bytes + it->second <= POOL_BYTES) {
-            pool_kept.push_back({p, it->second});
+            pool_kept[pool_nkept++] = {p, it->second};
             pool_kept_bytes += it->second;
             pool_live.erase(it);
             return;

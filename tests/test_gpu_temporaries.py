@@ -42,3 +42,19 @@ def test_kept_memory_is_given_back(hip):
         assert_ell_identical(g, got[0], "before and after the release")
     ref = orc.ab(A, A, M, 1e-6)
     np.testing.assert_array_equal(got[0].nnz, ref.nnz)
+
+
+def test_more_blocks_than_are_kept(hip):
+    """Temporaries past the number that is kept (64) are freed; those kept are
+    handed out again, each to one caller."""
+    lib = hip.lib()
+    for _ in range(2):
+        held = []
+        for k in range(80):
+            p = C.c_void_p()
+            assert lib.bmlhip_temp_malloc(C.byref(p), C.c_size_t(1000 * (k % 7) + k)) == 0
+            held.append(p.value)
+        assert len(set(held)) == 80
+        for p in held:
+            lib.bmlhip_temp_free(C.c_void_p(p))
+    hip.release_temporaries()
