@@ -1786,12 +1786,17 @@ __device__ __forceinline__ cf64 fx_scale(cf64 v, double sc) { return {v.x * sc, 
 // to 6 waves per SIMD (three blocks).  Double holds them to 4 (two blocks):
 // its 12-byte entries past the L2 are the bound, and three blocks a CU drift
 // further apart in X (437 GB a launch on the 32^3 SP2 step, at 7.2 TB/s) and
-// spill: 61.0 ms at 6, 47.6 at 4.  Complex blocks are LDS-bound at 1-2 per CU.
-template <typename T> struct WinbOcc { static constexpr int value = 1; };
-template <> struct WinbOcc<float> { static constexpr int value = 6; };
-template <> struct WinbOcc<double> { static constexpr int value = 4; };
+// spill: 61.0 ms at 6, 47.6 at 4.  Complex blocks leave LDS for two per CU,
+// which need 4: left to itself the compiler took 165 registers for the
+// unfused double product and 143 for the fused single step, and one block ran
+// (squares of 60000 rows of 300, 21.4 ms; now 14.1; 4-iteration solve of the
+// 18^3 lattice, single, 3.65 ms; now 2.61).  The fused double step spills 88
+// registers at 4 and is faster at 2 (3.9 ms against 4.3).
+template <typename T, bool FUSE> struct WinbOcc { static constexpr int value = 4; };
+template <bool FUSE> struct WinbOcc<float, FUSE> { static constexpr int value = 6; };
+template <> struct WinbOcc<cf64, true> { static constexpr int value = 1; };
 template <typename T, int W, int WB, int R, bool SYM, bool FUSE>
-__global__ __launch_bounds__(64 * W, WinbOcc<T>::value) void k_spgemm_winb(WinParams p) {
+__global__ __launch_bounds__(64 * W, (WinbOcc<T, FUSE>::value)) void k_spgemm_winb(WinParams p) {
     using E = Elem<T>;
     using F = FxW<T>;
     using V = typename F::V;
@@ -1983,7 +1988,8 @@ __global__ __launch_bounds__(64 * W, WinbOcc<T>::value) void k_spgemm_winb(WinPa
                 // 103 GB of entries past the L2 at 6.7 TB/s.  8 rows per
                 // block stream 70 GB and take as long (two blocks per CU);
                 // three rounds in flight and windows of 2^11 gain nothing.
-                constexpr int EPL = 4;
+                // (two a lane for 16-byte elements, whose registers are short)
+                constexpr int EPL = sizeof(T) > 8 ? 2 : 4;
                 constexpr unsigned ALL = (1u << R) - 1u;
                 struct Round {
                     int n;        // entries from the round's first to its segment's end
