@@ -1,7 +1,8 @@
 /*
  * Launch-shape choice for the ELLPACK row-product kernels.  The exact engine
- * takes the direct-index kernel where its index fits (pick_direct below);
- * what follows is the hash kernels' choice.
+ * takes the direct-index kernel where it is the faster one and its index fits
+ * (direct_wins and pick_direct below); what follows is the hash kernels'
+ * choice.
  *
  * group (lanes per output row) follows the length of the rows of B that a
  * step streams: a step holds three GROUP-wide chunks of a row of B in
@@ -87,9 +88,9 @@ static int direct_wins(size_t es, int span, int max_a, int max_b, long long est,
  * step.  W wavefronts per block and the blocks per CU follow the LDS: the
  * block needs 8 bytes per 32 reachable columns, and each row sizeof(T) + 2 per
  * column that any row of the block touches (15% more for each further row: on
- * a lattice a step along the fast axis adds the ball's cross-section; as many
- * again where up to 16 entries share a wavefront with other rows and are not
- * known to share columns with them); the W with the most wavefronts per CU is
+ * a lattice a step along the fast axis adds the ball's cross-section, near
+ * the diagonal less; as many again where up to 16 entries share a wavefront
+ * with other rows and are not known to share columns with them); the W with the most wavefronts per CU is
  * taken, the larger of equals (its rows share more of the index).  A block
  * whose rows touch more than that forms them in several passes; a row that
  * does not fit alone is left to the global-table pass.  Without a hint the

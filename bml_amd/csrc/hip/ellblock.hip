@@ -54,9 +54,9 @@ constexpr int EMPTY = -1;
 constexpr int NUM_WAVES = BMLHIP_EB_WAVES;  // wavefronts per block row in k_eb_numeric
 // pairs per batch, the unit of work a wavefront of k_eb_numeric claims: batch
 // k holds the slots whose first pair lies in [EB_BATCH k, EB_BATCH (k+1)).
-// 16 against 32: 1.44 against 1.47 ms (FP64), 0.85 against 0.90 ms (FP32)
-// for the symmetric X^2 of the 16x16x8-site, 32-orbital lattice; 2 or 8
-// wavefronts per block row ran 10-20% slower than 4.
+// 16 against 32: 0.85 against 0.90 ms (FP32) for the symmetric X^2 of the
+// 16x16x8-site, 32-orbital lattice; 2 or 8 wavefronts per block row ran 10-20%
+// slower than 4.
 constexpr int EB_BATCH = BMLHIP_EB_BATCH;
 constexpr int STREAM_BATCH = 8;  // and for k_eb_stream (see there)
 constexpr int EB_QUEUES = 8;  // k_eb_stream: one queue of batches per XCD,
@@ -1172,20 +1172,21 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
 // What bounds it is the L2 misses of the tiles: 16 KB per pair of tiles, and
 // few tiles are met twice by one workgroup.  With a workgroup per block row
 // (the FP32 and bf16 kernel above) 64 rows were at work on an XCD at a time
-// and 78% of the reads missed its L2, 16 GB at 7 TB/s for the general X^2 of
-// the 16x16x8-site, 32-orbital lattice (1.25 M pairs).  Here workgroups stay
+// and 78% of the reads missed its L2, 16.2 GB at 7.1 TB/s for the general X^2
+// of the 16x16x8-site, 32-orbital lattice (1.25 M pairs).  Here workgroups stay
 // for the whole product and their wavefronts take batches (about STREAM_BATCH
 // pairs, whole slots of one block row) from 8 queues, one per XCD, each an
 // eighth of all batches in block row order: 3 to 7 rows are at work on an
-// XCD, their left tiles stay in its L2, and 45% of the reads miss.  A
+// XCD, their left tiles stay in its L2, and 45% of the reads miss (9.2 GB).  A
 // wavefront whose queue is empty goes on to the next one, so no CU waits for
-// the longest row.  That product: 2.27 -> 1.75 ms with its compaction at
-// 0.11 (matrix cores busy 1.2 ms); the fused symmetric update of the
-// 8x8x6-site lattice (384 block rows, 125 k pairs): 325 -> 240 us.
+// the longest row.  That product: 2.27 ms with the compaction inside it ->
+// 1.87 and 0.11 for the compaction (matrix cores busy 1.2 ms); the fused
+// symmetric update of the 8x8x6-site lattice (384 block rows, 125 k pairs):
+// 325 -> 248 us.
 //
-// Batches of 8 pairs: the X^2 2.13 ms, the 25 updates of an SP2 loop on the
-// 8x8x6 lattice 7.5 ms; of 16, 2.13 and 7.9; of 32, 2.24 and 8.3; of 4, 2.20
-// and 7.7.  A wavefront's first batch is its own number, not a claim, and a
+// Batches of 8 pairs: the whole x2 call with a copy of its result 2.13 ms, an
+// SP2 solve of 25 updates on the 8x8x6 lattice 7.5 ms; of 16, 2.13 and 7.9; of
+// 32, 2.24 and 8.3; of 4, 2.20 and 7.7.  A wavefront's first batch is its own number, not a claim, and a
 // workgroup asks no queue that it has found empty: 2048 wavefronts that each
 // asked all 8 heads spent 150 us of the update on those atomics.  Three
 // workgroups per CU spill and miss more (2.97 ms), one leaves the matrix
@@ -1843,7 +1844,10 @@ __global__ __launch_bounds__(256) void k_eb_trace_frob(int NB, int MB, const T *
 // the fused SP2 product's three sums over its block rows or workgroups (next
 // tr X, next tr X^2, and |X - X^2|^2) into status scalars 0, 1, 2: one block
 // of 1024 threads, each sum over a fixed partition and a fixed tree (one
-// launch, not three)
+// launch, not three).  What it adds up is not of a fixed order: a lane's part
+// holds the slots that its wavefront claimed, of one block row (k_eb_numeric)
+// or of any (k_eb_stream), so the sums may differ in the last bits from run to
+// run
 __global__ __launch_bounds__(1024) void k_eb_sum3(const double *x, int n, bmlhip_status *st,
                                                   const int *skip) {
     __shared__ double part[1024];

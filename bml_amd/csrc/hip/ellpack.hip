@@ -1,6 +1,6 @@
 // gfx950 kernels for the ELLPACK-R thresholded multiply path: the hash-table
-// products (the exact engine's direct-index kernel, which takes most
-// products, is rowdir.hip), the unordered and window engines, the adds and
+// products (the exact engine's direct-index kernel, which takes most products
+// of up to 2^14 columns and of longer rows, is rowdir.hip), the unordered and window engines, the adds and
 // the single-pass kernels.
 //
 // Row accumulator of the hash kernels.  Every output row is built by a "group" of GROUP lanes
@@ -1980,12 +1980,12 @@ __global__ __launch_bounds__(64 * W, (WinbOcc<T, FUSE>::value)) void k_spgemm_wi
                 // arithmetic, and a round that does not exist is loaded from
                 // an empty one, so that the loads are straight-line code and
                 // the adds wait only for their own.  Products are counted per
-                // lane when a group is read, not per segment.  Together 9.7
-                // vector and 10 scalar instructions per wavefront's atomic
-                // came down to 5.5 and 6, and the product of the 24^3
-                // lattice's iterate from 16.8 to 15.1 ms: what is left is
-                // the atomics themselves (about 9 of 11.8 clocks each) and
-                // 103 GB of entries past the L2 at 6.7 TB/s.  8 rows per
+                // lane when a group is read, not per segment.  Together 9.5
+                // vector and 9.8 scalar instructions per wavefront's atomic
+                // came down to 5.5 and 5.8, and the product of the 24^3
+                // lattice's iterate from 17.4 to 14.7 ms: what is left is
+                // the atomics themselves (6.3 clocks of LDS each, of 11.4)
+                // and 100 GB of entries past the L2 at 6.8 TB/s.  8 rows per
                 // block stream 70 GB and take as long (two blocks per CU);
                 // three rounds in flight and windows of 2^11 gain nothing.
                 // (two a lane for 16-byte elements, whose registers are short)

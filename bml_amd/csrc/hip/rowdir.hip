@@ -1,5 +1,6 @@
-// Row products on directly indexed accumulators: the exact engine's kernel
-// for all but very wide matrices.
+// Row products on directly indexed accumulators: the exact engine's kernel up
+// to 2^14 columns and, above, for long rows and for rows that share columns
+// (the line is direct_wins in bml_hip_tune.c).
 //
 // W wavefronts of a block form RB = W * 64/GROUP consecutive output rows, a
 // group of GROUP lanes per row (wavefronts beyond W help with steps 1 to 3
@@ -28,7 +29,8 @@
 // the next rank in (jp, kp) order by a ballot prefix count.  Rows therefore
 // come out with the sums and the column order of a sequential walk.
 //
-// Measured on one MI355X against the hash-table kernels (double unless said):
+// Measured on one MI355X against the hash-table kernels (double unless said;
+// the cases below the line are beside it):
 // 32^3 lattice iterate squared (177 entries a row, 1.03e9 products) 4.71 ->
 // 1.81 ms (1.94 without helpers); 24^3 complex double (279 a row, 1.08e9
 // products) 10.5 -> 5.5 ms (6.7);
