@@ -302,7 +302,8 @@ def ellblock_sp2(hip, G):
                 continue
             flops = 2.0 * 32 ** 3 * prof.products[p]
             tf = flops / (prof.kernel_ms[p] * 1e-3) / 1e12
-            entry[f"x2_{key}"] = {"kernel": "k_eb_numeric", "launches": n,
+            entry[f"x2_{key}"] = {"kernel": "k_eb_stream" if p == 2 else "k_eb_numeric",
+                                  "launches": n,
                                   "avg_launch_ms": round(prof.kernel_ms[p] / n, 4),
                                   "block_pairs_per_launch": int(prof.products[p] / n),
                                   "tflops": round(tf, 2), "mfma_peak_tflops": MFMA_PEAK_TFLOPS[key],
