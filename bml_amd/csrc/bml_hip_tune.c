@@ -60,11 +60,17 @@
  * - up to 32 entries, several rows to a wavefront: only on rows known to
  *   share columns (fewer distinct ones than 7/10 of the products), up to
  *   2^17 columns and 350 for each product of a row (48^3 lattice: 25 a row
- *   875 and 690, 7 a row 151 and 333; all over, N = 32000, 12: 148 and 269). */
-static int direct_wins(size_t es, int span, int max_a, int max_b, long long est, int known)
+ *   875 and 690, 7 a row 151 and 333; all over, N = 32000, 12: 148 and 269).
+ *
+ * A solve's iterate that has not been squared yet: direct up to 2^17 columns.
+ * The shape serves until the counts are polled, and the rows grow meanwhile
+ * (five systems of up to 27000 rows, a poll every 3 iterations: 117 ms, with
+ * the hash kernels until the first poll 167). */
+static int direct_wins(size_t es, int span, int max_a, int max_b, long long est, int known,
+                       int solve)
 {
     const long long products = (long long) max_a * max_b;
-    if (span <= 16384)
+    if (span <= 16384 || (solve && !known && span <= 131072))
         return 1;
     const int shared = known && 10 * est <= 7 * products;
     if (max_b > 64)
@@ -98,13 +104,16 @@ static int direct_wins(size_t es, int span, int max_a, int max_b, long long est,
  * are provided for, 6500 for rows of more than 64 entries, whose hash tables
  * held as many (double, N = 16384, 80 entries all over: 20.8 ms with 3000,
  * 4.2 with 6500, the hash kernel 8.7; near the diagonal 0.99, 1.75, 5.3).
+ * solve: the rows are a solve's first iterate, far shorter than max_a, and
+ * 3000 columns serve them and what grows from them until they are known (32^3
+ * lattice, M = 256: 334 us, with 6500 606).
  * Rows so short that all columns fit are indexed by the column itself.
  * waves != 0 asks for the shape of that many wavefronts per block (the
  * autotuner's candidates; fewer rows than CUs then do not rule it out). */
 static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long long est,
-                       int known, int grows, int waves, bmlh_spgemm_shape *out)
+                       int known, int grows, int solve, int waves, bmlh_spgemm_shape *out)
 {
-    if (N <= 0 || span <= 0 || !direct_wins(es, span, max_a, max_b, est, known))
+    if (N <= 0 || span <= 0 || !direct_wins(es, span, max_a, max_b, est, known, solve))
         return 0;
     int g = 8;
     while (g < 64 && (g < max_b || (long long) N * g < 64 * 2048))
@@ -123,14 +132,14 @@ static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long lo
         est = span;
     const long long per = (long long) es + 2;
     const int dense = span * per <= 6 * 1024 || (2 * est >= span && span * per <= 20 * 1024);
-    const int shared = known && 10 * est <= 7 * (long long) max_a * max_b;
+    const int shared = known ? 10 * est <= 7 * (long long) max_a * max_b : solve;
     const long long words = span / 32 + 2;
     const long long cu = 160 * 1024;
     if (!known) {
         /* at most what the LDS holds beside the index */
         const long long room = (cu - 8 * words - 64 * (long long) es - 192) /
                                    (per + (span > 65536 ? 4 : 0)) - 40;
-        long long most = max_b > 64 ? 6500 : 3000;
+        long long most = max_b > 64 && !solve ? 6500 : 3000;
         if (most > room)
             most = room;
         if (most < 3000)
@@ -380,7 +389,8 @@ static void pick(int precision, int N, int span, int max_a, int max_b, int touch
      * so is a batch's work queue) */
     if (engine == BMLHIP_ROW_EXACT && !(flags & BMLH_PICK_QUEUE) && !shape_from_env())
         pick_direct(bmlh_elem_size(precision), N, span, max_a, max_b, est, touched_hint > 0,
-                    touched_hint > 0 && 20 * max_a > 21 * hint_max_a, direct_waves, out);
+                    touched_hint > 0 && 20 * max_a > 21 * hint_max_a, flags & BMLH_PICK_SOLVE,
+                    direct_waves, out);
 }
 
 void bmlh_pick_spgemm(int precision, int N, int span, int max_a, int max_b, int touched_hint,
@@ -558,7 +568,7 @@ void bmlh_tuned_spgemm(int precision, int N, int max_a, int max_b, int touched_h
     tune_load();
     char key[128];
     snprintf(key, sizeof key, "cu%d:p%d:f%d:e%d:n%d:a%d:b%d:t%d", bmlhip_device_cus(), precision,
-             flags, out->engine, qbucket(N), qbucket(max_a), qbucket(max_b),
+             flags & (BMLH_PICK_SQUARE | BMLH_PICK_EXACT), out->engine, qbucket(N), qbucket(max_a), qbucket(max_b),
              qbucket(touched_hint));
     for (int k = 0; k < g_ntab; k++)
         if (!strcmp(g_tab[k].key, key)) {

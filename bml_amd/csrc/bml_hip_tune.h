@@ -24,6 +24,8 @@ typedef struct bmlh_spgemm_shape {
  * SP2 iterations), the only one the window engine takes. */
 #define BMLH_PICK_SQUARE 1
 #define BMLH_PICK_EXACT 2
+#define BMLH_PICK_SOLVE 8 /* a solve's iterate: before the first product is
+                             known, max_a is what its rows may grow to */
 #define BMLH_PICK_QUEUE 4 /* the rows come from a batch's work queue, which
                              only the hash kernels take them from */
 void bmlh_pick_spgemm(int precision, int N, int span, int max_a, int max_b, int touched_hint,

@@ -115,7 +115,8 @@ static void sp2_shape(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpack_hip_t **X2
                    : X->aux->len_hint > 0 && X->aux->len_hint < X->M ? X->aux->len_hint : X->M;
     sp2_tune_ctx c = { X, X2p, threshold, sym };
     bmlh_tuned_spgemm(X->matrix_precision, X->N, mx, mx, X->aux->touched_hint,
-                      X->aux->hint_max_nnz, BMLH_PICK_SQUARE, sh, measure_sp2, &c);
+                      X->aux->hint_max_nnz, BMLH_PICK_SQUARE | BMLH_PICK_SOLVE, sh, measure_sp2,
+                      &c);
 }
 
 static int same_shape(const bmlh_spgemm_shape *a, const bmlh_spgemm_shape *b)
@@ -634,7 +635,8 @@ void bml_hip_sp2_ellpack_batch(int nsys, bml_matrix_ellpack_hip_t *const *H,
         const int mx = cur->aux->stats_valid ? cur->aux->max_nnz : cur->M;
         bmlh_spgemm_shape sh;
         bmlh_pick_spgemm(cur->matrix_precision, N, span, mx, mx, touched, hint_max,
-                         BMLH_PICK_SQUARE | (d.b.d_list ? BMLH_PICK_QUEUE : 0), &sh);
+                         BMLH_PICK_SQUARE | BMLH_PICK_SOLVE | (d.b.d_list ? BMLH_PICK_QUEUE : 0),
+                         &sh);
         if (o.graph) {
             /* replay the iteration as a graph; capture anew when the launch
              * shape or the precision changes (the first pass runs eagerly so

@@ -202,3 +202,19 @@ def test_lds_for_rows_not_known_to_share_columns(prec):
         rb = sh.waves * (64 // sh.group)
         assert sh.engine == DIRECT and sh.group <= 16
         assert rows_held(prec, sh, rb * (touched or n * n)) >= rb, (N, n, sh.key())
+
+
+@pytest.mark.parametrize("prec", sorted(ELEM))
+@pytest.mark.parametrize("N,n", [(576, 256), (20000, 9), (48000, 7), (110592, 256), (3000, 8)])
+def test_first_iterate_of_a_solve(prec, N, n):
+    """A solve's iterate before its first product is known: the direct kernel
+    up to 2^17 columns, with LDS for 3000 columns at most, and the cache key
+    of any other square."""
+    solve = 8
+    sh, x2 = Shape(), analytic(prec, N, n)
+    hip.lib().bmlh_pick_spgemm(prec, N, N, n, n, 0, 0, SQUARE | solve, C.byref(sh))
+    assert sh.engine == DIRECT and sh.wrows == N
+    if x2.engine == DIRECT:
+        assert sh.table <= x2.table
+    hip.lib().bmlh_pick_spgemm(prec, 262144, 262144, 9, 9, 0, 0, SQUARE | solve, C.byref(sh))
+    assert sh.engine == EXACT
