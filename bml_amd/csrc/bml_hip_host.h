@@ -16,7 +16,8 @@ struct bml_hip_aux {
     int max_nnz;
     long long total_nnz;
     int touched_hint;      /* distinct columns per row seen the last time this
-                              matrix was squared (0 = unknown) */
+                              matrix was squared (0 = unknown; negative: of
+                              the matrix that this one was made from) */
     int hint_max_nnz;      /* its longest row at that time */
     int temp;              /* a call's temporary: arrays from bmlhip_temp_malloc
                               (an ellblock's bsize is another matrix's) */
@@ -58,6 +59,8 @@ void bmlh_put_scalar(int prec, double s, void *buf);
 struct bml_hip_aux *bmlh_aux_new(void);
 /* the row statistics no longer hold: rows may have grown by `more` entries */
 void bmlh_stats_stale(struct bml_hip_aux *aux, int more);
+/* the matrix changed: its count of distinct columns is an earlier one's */
+void bmlh_hint_stale(struct bml_hip_aux *aux);
 /* dst's rows are copies of src's */
 void bmlh_copy_stats(struct bml_hip_aux *dst, const struct bml_hip_aux *src);
 void bmlh_set_stats(struct bml_hip_aux *aux, const bmlhip_status *st);

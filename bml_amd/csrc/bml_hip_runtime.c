@@ -155,6 +155,12 @@ void bmlh_copy_stats(struct bml_hip_aux *dst, const struct bml_hip_aux *src)
     dst->temp = temp;
 }
 
+void bmlh_hint_stale(struct bml_hip_aux *aux)
+{
+    if (aux->touched_hint > 0)
+        aux->touched_hint = -aux->touched_hint;
+}
+
 void bmlh_stats_stale(struct bml_hip_aux *aux, int more)
 {
     if (aux->stats_valid)

@@ -104,16 +104,22 @@ static int direct_wins(size_t es, int span, int max_a, int max_b, long long est,
  * are provided for, 6500 for rows of more than 64 entries, whose hash tables
  * held as many (double, N = 16384, 80 entries all over: 20.8 ms with 3000,
  * 4.2 with 6500, the hash kernel 8.7; near the diagonal 0.99, 1.75, 5.3).
- * solve: the rows are a solve's first iterate, far shorter than max_a, and
+ * seen: the distinct columns to expect from the count of the matrix that this
+ * one was made from (a client's loop of x2 and add_norm), 0 without one; the
+ * LDS is for 9/8 of them, or 3000.  solve: the rows are a solve's first iterate, far shorter than max_a, and
  * 3000 columns serve them and what grows from them until they are known (32^3
  * lattice, M = 256: 334 us, with 6500 606).
  * Rows so short that all columns fit are indexed by the column itself.
  * waves != 0 asks for the shape of that many wavefronts per block (the
  * autotuner's candidates; fewer rows than CUs then do not rule it out). */
 static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long long est,
-                       int known, int grows, int solve, int waves, bmlh_spgemm_shape *out)
+                       int known, long long seen, int grows, int solve, int waves,
+                       bmlh_spgemm_shape *out)
 {
-    if (N <= 0 || span <= 0 || !direct_wins(es, span, max_a, max_b, est, known, solve))
+    if (N <= 0 || span <= 0)
+        return 0;
+    if (!direct_wins(es, span, max_a, max_b, est, known, solve) &&
+        !(seen && max_b <= 64 && direct_wins(es, span, max_a, max_b, seen, 1, solve)))
         return 0;
     int g = 8;
     while (g < 64 && (g < max_b || (long long) N * g < 64 * 2048))
@@ -132,14 +138,15 @@ static int pick_direct(size_t es, int N, int span, int max_a, int max_b, long lo
         est = span;
     const long long per = (long long) es + 2;
     const int dense = span * per <= 6 * 1024 || (2 * est >= span && span * per <= 20 * 1024);
-    const int shared = known ? 10 * est <= 7 * (long long) max_a * max_b : solve;
+    const int shared = known || seen ? 10 * (known ? est : seen) <= 7 * (long long) max_a * max_b
+                                     : solve;
     const long long words = span / 32 + 2;
     const long long cu = 160 * 1024;
     if (!known) {
         /* at most what the LDS holds beside the index */
         const long long room = (cu - 8 * words - 64 * (long long) es - 192) /
                                    (per + (span > 65536 ? 4 : 0)) - 40;
-        long long most = max_b > 64 && !solve ? 6500 : 3000;
+        long long most = seen ? seen * 9 / 8 : (max_b > 64 && !solve ? 6500 : 3000);
         if (most > room)
             most = room;
         if (most < 3000)
@@ -207,6 +214,15 @@ static int shape_from_env(void)
     return 0;
 }
 
+/* The distinct columns of a row when rows of up to hint_max_a entries had
+ * `touched`: they grow about as the rows' length does. */
+static long long distinct(int touched, int max_a, int hint_max_a, long long bound)
+{
+    const double grow = hint_max_a > 0 && max_a > hint_max_a ? (double) max_a / hint_max_a : 1.0;
+    const long long est = (long long) (touched * grow) + 1;
+    return est > bound ? bound : est;
+}
+
 /* bmlh_pick_spgemm; direct_waves != 0: where it takes the direct kernel, its
  * shape of that many wavefronts per block */
 static void pick(int precision, int N, int span, int max_a, int max_b, int touched_hint,
@@ -220,14 +236,8 @@ static void pick(int precision, int N, int span, int max_a, int max_b, int touch
     if (bound > N)
         bound = N;
     long long est = bound;
-    if (touched_hint > 0) {
-        /* the rows grew since the hint was taken: a row's distinct count
-         * grows about as its length */
-        double grow = hint_max_a > 0 && max_a > hint_max_a ? (double) max_a / hint_max_a : 1.0;
-        est = (long long) (touched_hint * grow) + 1;
-        if (est > bound)
-            est = bound;
-    }
+    if (touched_hint > 0)
+        est = distinct(touched_hint, max_a, hint_max_a, bound);
     long long need = est * 3 / 2;
     if (need < est + max_b)
         need = est + max_b;
@@ -389,6 +399,7 @@ static void pick(int precision, int N, int span, int max_a, int max_b, int touch
      * so is a batch's work queue) */
     if (engine == BMLHIP_ROW_EXACT && !(flags & BMLH_PICK_QUEUE) && !shape_from_env())
         pick_direct(bmlh_elem_size(precision), N, span, max_a, max_b, est, touched_hint > 0,
+                    touched_hint < 0 ? distinct(-touched_hint, max_a, hint_max_a, bound) : 0,
                     touched_hint > 0 && 20 * max_a > 21 * hint_max_a, flags & BMLH_PICK_SOLVE,
                     direct_waves, out);
 }

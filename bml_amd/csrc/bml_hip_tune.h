@@ -17,8 +17,8 @@ typedef struct bmlh_spgemm_shape {
 
 /* Launch shape for a product whose left rows hold up to max_a entries and
  * right rows up to max_b; touched_hint is the largest distinct-column count
- * seen the last time (0 = unknown), when the left rows held up to
- * hint_max_a entries.  span: the columns 64 consecutive rows can reach (N,
+ * seen the last time (0 = unknown; negative: seen with the matrix that this
+ * one was made from), when the left rows held up to hint_max_a entries.  span: the columns 64 consecutive rows can reach (N,
  * less for block-diagonal batches).  The engine follows bml_hip_set_row_engine unless
  * flags holds BMLH_PICK_EXACT; BMLH_PICK_SQUARE marks a product X*X (x2, the
  * SP2 iterations), the only one the window engine takes. */

@@ -515,6 +515,8 @@ void *bml_multiply_x2_ellpack_hip(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpac
     bmlh_set_stats(X2->aux, &st);
     X->aux->touched_hint = st.max_touched;
     X->aux->hint_max_nnz = max_nnz_of(X);
+    X2->aux->touched_hint = -st.max_touched;
+    X2->aux->hint_max_nnz = X->aux->hint_max_nnz;
     double *trace = malloc(2 * sizeof(double));
     if (!trace) {
         bmlh_error(BML_HIP_ERR_ALLOC, "%s: host allocation failed", what);
@@ -551,6 +553,8 @@ void bml_multiply_x2_ellpack_hip_noalloc(bml_matrix_ellpack_hip_t *X,
     bmlh_set_stats(X2->aux, &st);
     X->aux->touched_hint = st.max_touched;
     X->aux->hint_max_nnz = max_nnz_of(X);
+    X2->aux->touched_hint = -st.max_touched;
+    X2->aux->hint_max_nnz = X->aux->hint_max_nnz;
     traces[0] = st.scalars[0];
     traces[1] = st.scalars[1];
 }
@@ -622,7 +626,7 @@ static void add_impl(bml_matrix_ellpack_hip_t *A, bml_matrix_ellpack_hip_t *B, d
     } else {
         finish_into(what, A);
     }
-    A->aux->touched_hint = 0;
+    bmlh_hint_stale(A->aux);
 }
 
 void bml_add_ellpack_hip(bml_matrix_ellpack_hip_t *A, bml_matrix_ellpack_hip_t *B, double alpha,
@@ -737,7 +741,7 @@ void bml_threshold_ellpack_hip(bml_matrix_ellpack_hip_t *A, double threshold)
     bmlhip_status st;
     bmlh_finish(what, &st);
     bmlh_stats_stale(A->aux, 0);
-    A->aux->touched_hint = 0;
+    bmlh_hint_stale(A->aux);
 }
 
 bml_matrix_ellpack_hip_t *bml_threshold_new_ellpack_hip(const bml_matrix_ellpack_hip_t *A,

@@ -218,3 +218,26 @@ def test_first_iterate_of_a_solve(prec, N, n):
         assert sh.table <= x2.table
     hip.lib().bmlh_pick_spgemm(prec, 262144, 262144, 9, 9, 0, 0, SQUARE | solve, C.byref(sh))
     assert sh.engine == EXACT
+
+
+def test_count_of_the_matrix_it_was_made_from():
+    """A negative count is an earlier matrix's (before an add, or the factor
+    of a square): LDS for the columns to expect by it, and the crossover's side
+    of rows that share columns."""
+    def pick(prec, N, n, touched, hint):
+        sh = Shape()
+        hip.lib().bmlh_pick_spgemm(prec, N, N, n, n, touched, hint, SQUARE, C.byref(sh))
+        return sh
+
+    never, seen = pick(DOUBLE, 32768, 148, 0, 0), pick(DOUBLE, 32768, 148, -1100, 140)
+    assert never.engine == seen.engine == DIRECT
+    assert rows_held(DOUBLE, never, 6500) >= 1
+    # rows in flight per CU: the LDS is not kept for 6500 columns a row
+    assert seen.waves * (160 * 1024 // seen.table) > never.waves * (160 * 1024 // never.table)
+    wide = pick(DOUBLE, 16384, 80, -5300, 80)
+    assert wide.engine == DIRECT and rows_held(DOUBLE, wide, 5300) >= 1
+    grown = pick(DOUBLE, 16384, 88, -5300, 80)
+    assert grown.engine == DIRECT and rows_held(DOUBLE, grown, 5830) >= 1
+    assert pick(DOUBLE, 32768, 25, 0, 0).engine == EXACT
+    assert pick(DOUBLE, 32768, 25, -90, 25).engine == DIRECT
+    assert pick(DOUBLE, 32768, 25, -600, 25).engine == EXACT
