@@ -497,6 +497,16 @@ static int run_product(bml_matrix_ellpack_hip_t *A, bml_matrix_ellpack_hip_t *B,
     return run_product_ws(A, B, C, threshold, kind, hint_owner, NULL, 0, NULL, what);
 }
 
+/* X2 is X's square: until it has been squared itself (a count of that stays),
+ * X's count tells what its rows may touch */
+static void hint_of_square(struct bml_hip_aux *x2, const struct bml_hip_aux *x)
+{
+    if (x2->touched_hint > 0)
+        return;
+    x2->touched_hint = -x->touched_hint;
+    x2->hint_max_nnz = x->hint_max_nnz;
+}
+
 void *bml_multiply_x2_ellpack_hip(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpack_hip_t *X2,
                                   double threshold)
 {
@@ -515,8 +525,7 @@ void *bml_multiply_x2_ellpack_hip(bml_matrix_ellpack_hip_t *X, bml_matrix_ellpac
     bmlh_set_stats(X2->aux, &st);
     X->aux->touched_hint = st.max_touched;
     X->aux->hint_max_nnz = max_nnz_of(X);
-    X2->aux->touched_hint = -st.max_touched;
-    X2->aux->hint_max_nnz = X->aux->hint_max_nnz;
+    hint_of_square(X2->aux, X->aux);
     double *trace = malloc(2 * sizeof(double));
     if (!trace) {
         bmlh_error(BML_HIP_ERR_ALLOC, "%s: host allocation failed", what);
@@ -553,8 +562,7 @@ void bml_multiply_x2_ellpack_hip_noalloc(bml_matrix_ellpack_hip_t *X,
     bmlh_set_stats(X2->aux, &st);
     X->aux->touched_hint = st.max_touched;
     X->aux->hint_max_nnz = max_nnz_of(X);
-    X2->aux->touched_hint = -st.max_touched;
-    X2->aux->hint_max_nnz = X->aux->hint_max_nnz;
+    hint_of_square(X2->aux, X->aux);
     traces[0] = st.scalars[0];
     traces[1] = st.scalars[1];
 }
