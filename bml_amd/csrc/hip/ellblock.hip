@@ -1179,10 +1179,10 @@ __global__ __launch_bounds__(64 * NUM_WAVES, (EbOcc<T, ENGINE>::value)) void k_e
 // eighth of all batches in block row order: 3 to 7 rows are at work on an
 // XCD, their left tiles stay in its L2, and 45% of the reads miss (9.2 GB).  A
 // wavefront whose queue is empty goes on to the next one, so no CU waits for
-// the longest row.  That product: 2.27 ms with the compaction inside it ->
-// 1.87 and 0.11 for the compaction (matrix cores busy 1.2 ms); the fused
-// symmetric update of the 8x8x6-site lattice (384 block rows, 125 k pairs):
-// 325 -> 248 us.
+// the longest row.  That product with its compaction: 2.27 -> 1.83 ms (events
+// over 20 calls; in a kernel trace 1.87 and 0.11, matrix cores busy 1.2); the
+// fused symmetric update of the 8x8x6-site lattice (384 block rows, 125 k
+// pairs): 325 -> 248 us (trace, the full iterates).
 //
 // Batches of 8 pairs: the whole x2 call with a copy of its result 2.13 ms, an
 // SP2 solve of 25 updates on the 8x8x6 lattice 7.5 ms; of 16, 2.13 and 7.9; of
